@@ -40,13 +40,8 @@ int hip_fail(hipError_t e, const char* where) {
 void clear_pending_error() { (void)hipGetLastError(); }
 
 int elem_bytes(int32_t dt) { return dt == PKV_F32 ? 4 : dt == PKV_FP8_E4M3 ? 1 : 2; }
-// Nonzero finite scale whose reciprocal is exact: a power of two whose
-// inverse is a normal float.
-bool exact_reciprocal(float s) {
-  int e = 0;
-  const float m = std::frexp(s, &e);
-  return std::isfinite(s) && (m == 0.5f || m == -0.5f) && e > -125 && e < 127;
-}
+// Scales for which the append's corrected division (pkv_fp8.h) is exact.
+bool fast_scale(float s) { return std::fabs(s) >= 0x1p-60f && std::fabs(s) <= 0x1p60f; }
 bool valid_dtype(int32_t dt) { return dt == PKV_F32 || dt == PKV_F16 || dt == PKV_BF16; }
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
@@ -207,9 +202,9 @@ int pkv_reshape_and_cache(const void* key, const void* value, void* key_cache, v
   p.cache_dtype = cache_dtype;
   p.k_scale = k_scale;
   p.v_scale = v_scale;
-  p.scales_pow2 = exact_reciprocal(k_scale) && exact_reciprocal(v_scale);
-  p.k_inv = p.scales_pow2 ? 1.f / k_scale : 0.f;
-  p.v_inv = p.scales_pow2 ? 1.f / v_scale : 0.f;
+  p.fast_div = fp8 && fast_scale(k_scale) && fast_scale(v_scale);
+  p.k_inv = p.fast_div ? 1.f / k_scale : 0.f;
+  p.v_inv = p.fast_div ? 1.f / v_scale : 0.f;
   clear_pending_error();
   const hipError_t e = pkv::launch_reshape_and_cache(p, aligned, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "reshape_and_cache launch");

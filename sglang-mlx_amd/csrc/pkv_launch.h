@@ -43,11 +43,11 @@ struct RacParams {
   int32_t layout;  // 0 = paged 5-D, 1 = token-major
   int32_t kv_dtype;
   int32_t cache_dtype;
-  // FP8 caches store encode(x / scale); a power-of-two scale multiplies by
-  // its exact reciprocal instead (the same result, without a division).
+  // FP8 caches store encode(x / scale).  k_inv, v_inv: the rounded
+  // reciprocals; fast_div: both scales lie in [2^-60, 2^60] (pkv_fp8.h).
   float k_scale, v_scale;
   float k_inv, v_inv;
-  int32_t scales_pow2;
+  int32_t fast_div;
   // Set by launch_reshape_and_cache: the call writes at least
   // kRacStreamKBytes of K, so the paged layout's per-token K stores are
   // nontemporal (reshape_and_cache.hip).

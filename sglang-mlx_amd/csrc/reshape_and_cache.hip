@@ -8,12 +8,13 @@
 // (:9-12): identical types copy bits, float -> f16/bf16 rounds to nearest even.
 //
 // Two layouts:
-//  * paged 5-D: K [nb, H, D/x, bs, x], V [nb, H, D, bs].  One wavefront per
-//    (token, head): K leaves as D/x 16-byte chunks at a stride of bs*16 bytes,
-//    V as D single elements at a stride of bs elements (the layout makes V
-//    token-minor, so one token's stores cannot be wider than one element).
-//    Tokens that together fill a whole block in order (a prefill) instead
-//    write slices of the block's regions as whole lines (below).
+//  * paged 5-D: K [nb, H, D/x, bs, x], V [nb, H, D, bs].  One workgroup per
+//    window of bs batch tokens and head: tokens that together fill a whole
+//    block in order (a prefill) leave as whole lines; other tokens leave one
+//    (token, head) per wavefront, K as D/x 16-byte chunks at a stride of bs*16
+//    bytes, V as D single elements at a stride of bs elements (the layout
+//    makes V token-minor, so one token's stores cannot be wider than one
+//    element).
 //  * FP8 caches (E4M3 codes of x / scale, either layout): see below.
 //  * token-major (MHATokenPool / flash): K and V [num_slots, H, D].  A token's
 //    K row and V row are each one contiguous H*D run in both source and
@@ -21,6 +22,8 @@
 //    covers 1 KiB of one row.  Rows of at least 64 vectors go one token per
 //    wavefront with nontemporal stores; shorter rows one token per
 //    workgroup.
+#include <algorithm>
+
 #include "pkv_fp8.h"
 #include "pkv_launch.h"
 
@@ -65,75 +68,325 @@ __device__ __forceinline__ uint4 load_vec16(const typename Elem<S>::storage* __r
 }
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 
-// ---- paged 5-D layout, whole-block runs ------------------------------------------
-// When bs consecutive batch tokens write slots blk*bs .. blk*bs + bs - 1 in
-// order (a prefill writing whole blocks), the (block, head) region's K
-// ([D/8][bs][8]) and V ([D][bs]) are each one contiguous run of D*bs
-// elements that these tokens fill completely.  The wavefront of the run's
-// token at offset `off` then writes slice `off` of each region: elements
-// off*D .. off*D + D - 1, i.e. 16-byte units off*D/8 .. off*D/8 + D/8 - 1,
-// gathered from the run's source rows.  Every unit is written once and
-// whole, and the bs wavefronts of a run cover the region.  K unit u holds
-// dimensions 8c .. 8c+7 of token t (u = c*bs + t); V unit u holds tokens
-// 8g .. 8g+7 of dimension d (u = d*bs/8 + g).  The per-token path instead
-// writes a token's V as single 2-byte elements 2*bs bytes apart, each a
-// partial write of its line.  2-byte cache types (the kernel's ALIGNED
-// case).
+// ---- FP8 caches: E4M3 codes of x / scale (pkv_fp8.h) -------------------------------
+// Eight source elements -> eight codes.
+template <class KT>
+__device__ __forceinline__ uint2 encode8(const typename Elem<KT>::storage* __restrict__ src, const Fp8Scale& s) {
+  float v[8];
+  if constexpr (std::is_same<KT, F32>::value) {
+    const float4 a = reinterpret_cast<const float4*>(src)[0], b = reinterpret_cast<const float4*>(src)[1];
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  } else {
+    const uint4 w = *reinterpret_cast<const uint4*>(src);
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = to_f32<KT>((uint16_t)(u[i] & 0xffffu));
+      v[2 * i + 1] = to_f32<KT>((uint16_t)(u[i] >> 16));
+    }
+  }
+  return make_uint2(fp8_encode4_scaled(v, s), fp8_encode4_scaled(v + 4, s));
+}
+
+// ---- paged 5-D layout, windows of one block's tokens ------------------------------
+// One workgroup (or `parts` that share its tasks) per (window of BS
+// consecutive batch tokens, group of `hg` heads), for block sizes 8, 16 and
+// 32.  When BS consecutive batch tokens write slots blk*BS .. blk*BS + BS-1 in
+// order (a prefill writing whole blocks, a "run"), the (block, head) regions
+// of K ([D/x][BS][x]) and V ([D][BS]) are each one contiguous run of D*BS
+// elements that these tokens fill completely.  The workgroup of the window in which a run starts (at
+// most one run starts in BS consecutive tokens, as runs do not overlap)
+// writes both regions whole; the other tokens of the window, which lie
+// between the end of the previous window's run and the start of its own, are
+// written token by token.
 //
-// The slices' stores are nontemporal: each store instruction writes whole
-// lines that nothing in the launch reads back.  Measured on MI355X (same
-// box, one library per policy): the radix-shared workload's first decode
-// after its churn appends 84.0 -> 77.3 us per launch (the appends' lines no
-// longer linger in the caches), the reference's fp16 append at 1024
-// consecutive slots 4.33 -> 4.03 us, the churn append itself unchanged
-// (26.9 us).  The per-token path keeps default stores: its 2-byte V stores
-// rely on the L2 to combine them into lines (nontemporal, they made the
-// churn append 4.5x slower).
-template <class KT, class CT, int BS>
-__device__ __forceinline__ void rac_run_slice(const RacParams& p, int64_t first, int off, int head, int64_t blk,
-                                              int lane) {
-  using KS = typename Elem<KT>::storage;
-  using CS = typename Elem<CT>::storage;
-  static_assert(Elem<CT>::kBytes == 2 && BS % 8 == 0, "16-byte units of 2-byte elements");
-  constexpr int X = 8;
-  const int D = p.head_size;
-  const int per = D / X;  // units per wavefront and region
-  const int64_t slice = (blk * p.num_heads + head) * (int64_t)D * BS + (int64_t)off * per * X;
-  const int64_t hoff = (int64_t)head * D;
-  const KS* key = static_cast<const KS*>(p.key);
-  const KS* val = static_cast<const KS*>(p.value);
-  // Each lane moves two neighbouring elements of the slice: one store
-  // instruction writes 256 contiguous bytes of each region.
-  for (int i = 2 * lane; i < D; i += 128) {
-    const int u = off * per + i / X, e = i % X;
-    // K: dimensions 8c + e, +1 of token t.
-    const int c = u / BS, t = u % BS;
-    const KS* ks = key + (first + t) * p.key_stride + hoff + X * c + e;
-    // V: tokens 8g + e, +1 of dimension d.
-    const int d = u / (BS / X), g = u % (BS / X);
-    const KS* vs = val + (first + X * g + e) * p.value_stride + hoff + d;
-    const uint32_t kw = pack2(convert_elem<KT, CT>(ks[0]), convert_elem<KT, CT>(ks[1]));
-    const uint32_t vw = pack2(convert_elem<KT, CT>(vs[0]), convert_elem<KT, CT>(vs[p.value_stride]));
-    __builtin_nontemporal_store(kw, reinterpret_cast<uint32_t*>(static_cast<CS*>(p.key_cache) + slice + i));
-    __builtin_nontemporal_store(vw, reinterpret_cast<uint32_t*>(static_cast<CS*>(p.value_cache) + slice + i));
+// Run tasks, one per thread, eight elements of each region, index u:
+//   K: 16-bit caches: the 16-byte unit u = c*BS + t (dimensions 8c .. 8c+7 of
+//      token t), one 16-byte load of 8 source elements; FP8 caches: the
+//      8-byte half u of the units of 16 codes.
+//   V: u = (dim pair) * BS/4 + (token quad): two dimensions of four tokens in
+//      four loads; v_perm regroups them by dimension and one exchange with
+//      the neighbouring lane (the pair's other quad) leaves each lane eight
+//      tokens of one dimension, so 64 lanes store 1 KiB (FP8: 512 bytes) of
+//      the region in one piece.
+// Bound: HBM traffic.  Measured (ragged prompts of 97 .. 927 tokens, 8 heads
+// x 128, blocks of 16; passes back to back): 16,384 bf16 tokens 51.2 -> 22.4
+// us (134 MB, 6.0 TB/s), 8192 tokens into FP8 36.4 -> 13.9 us (50 MB; kernel
+// 38.2 -> 15.1 us under the profiler), against a wavefront per (token, head)
+// that gathered a 1/BS slice of each region with 2-byte loads: 131,072
+// wavefronts, and eight load instructions where one does.  The run stores are nontemporal: whole lines that
+// nothing in the launch reads back (a decode right after the append then
+// finds its own lines in the caches: radix-shared workload 84.0 -> 77.3 us
+// per launch).
+//
+// Per-token stores: a token's V elements lie BS elements apart, each store a
+// partial write of its line.  They keep the default policy, as the L2 combines
+// the tokens of a block into lines (nontemporal, they made the radix
+// workload's append 4.5x slower).  K chunks of a large call are stored
+// nontemporally (p.stream_k): a token's 16-byte chunks sit BS*16 bytes apart,
+// one per line, and a call writing more K than one XCD's L2 holds (4 MiB) has
+// its lines evicted before a later token fills their neighbours (4096 random
+// slots, 8 MiB of K: 76.4 -> 65.0 us).
+
+// Batch positions of a window that each wavefront needs: the run that started
+// in the previous window (prev) and the one that starts in this window (run),
+// -1 if there is none; every lane gets the same values.  slot: the slot of
+// token (window - 1) * BS + lane, -1 outside the batch.
+template <int BS>
+__device__ __forceinline__ void rac_window_runs(const RacParams& p, int64_t window, int lane, int64_t& prev,
+                                                int64_t& run, int& slot) {
+  const int64_t base = (window - 1) * BS;  // the lanes look at [base, base + 3 BS)
+  // Bit i: token base + i's slot is followed by its successor's.
+  auto links = [&](int64_t pos, int& slot) -> uint64_t {
+    slot = pos >= 0 && pos < p.num_tokens ? p.slot_mapping[pos] : -1;
+    const int next = pos >= 0 && pos + 1 < p.num_tokens ? p.slot_mapping[pos + 1] : -1;
+    return __ballot(slot >= 0 && slot < INT32_MAX && next == slot + 1);
+  };
+  int unused;
+  const uint64_t lo = links(base + lane, slot);
+  uint64_t follow = lo >> lane;
+  if constexpr (3 * BS > 64) {
+    const uint64_t hi = links(base + 64 + lane, unused);
+    if (lane > 0) follow |= hi << (64 - lane);
+  }
+  constexpr uint64_t kAll = ((uint64_t)1 << (BS - 1)) - 1;
+  const bool starts = lane < 2 * BS && slot >= 0 && slot % BS == 0 && (int64_t)slot + BS <= p.num_slots &&
+                      (follow & kAll) == kAll;
+  const uint64_t m = __ballot(starts);
+  constexpr uint64_t kWin = ((uint64_t)1 << BS) - 1;
+  const uint64_t mp = m & kWin, mr = (m >> BS) & kWin;
+  prev = mp ? base + __builtin_ctzll(mp) : -1;
+  run = mr ? base + BS + __builtin_ctzll(mr) : -1;
+}
+
+// Eight cache elements of a source run: one 16-byte vector (16-bit caches)
+// or 8 code bytes (FP8).
+template <class CT> struct Vec8 { using type = uint4; };
+template <> struct Vec8<FP8> { using type = uint2; };
+
+template <class KT, class CT>
+__device__ __forceinline__ typename Vec8<CT>::type load8(const typename Elem<KT>::storage* src, const Fp8Scale& s) {
+  if constexpr (std::is_same<CT, FP8>::value)
+    return encode8<KT>(src, s);
+  else
+    return load_vec16<KT, CT>(src);
+}
+
+template <bool NT> __device__ __forceinline__ void store8(void* dst, uint4 v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(dst));
+  else
+    *reinterpret_cast<uint4*>(dst) = v;
+}
+template <bool NT> __device__ __forceinline__ void store8(void* dst, uint2 v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x2_t, v), reinterpret_cast<u32x2_t*>(dst));
+  else
+    *reinterpret_cast<uint2*>(dst) = v;
+}
+
+// Two neighbouring source elements as floats (or raw 16-bit words when the
+// cache has the source's type).
+template <class KT> struct Pair { float a, b; };
+template <class KT>
+__device__ __forceinline__ Pair<KT> load_pair(const typename Elem<KT>::storage* src) {
+  if constexpr (std::is_same<KT, F32>::value) {
+    const float2 x = *reinterpret_cast<const float2*>(src);
+    return {x.x, x.y};
+  } else {
+    const uint32_t w = *reinterpret_cast<const uint32_t*>(src);
+    return {to_f32<KT>((uint16_t)(w & 0xffffu)), to_f32<KT>((uint16_t)(w >> 16))};
   }
 }
 
-// True when the token at batch position tok (slot `slot`, offset `off` in
-// its block) lies in a whole-block run: positions tok - off .. tok - off +
-// bs - 1 hold slots slot - off .. slot - off + bs - 1.  Wave-uniform; lanes
-// 0 .. bs-1 each check one entry.
-__device__ __forceinline__ bool rac_whole_block(const RacParams& p, int64_t tok, int32_t slot, int off, int lane) {
-  const int bs = p.block_size;
-  const int64_t first = tok - off;
-  if (first < 0 || first + bs > p.num_tokens) return false;
-  bool ok = true;
-  if (lane < bs) ok = p.slot_mapping[first + lane] == slot - off + lane;
-  return __all(ok);
+// A V task's four tokens of two dimensions -> eight tokens of one: this
+// lane's four of dimension d0 + (lane & 1) and its neighbour's.  (Both
+// dimensions are exchanged and the lane keeps one: the exchange then reads
+// registers as loaded, never a select's result.)
+__device__ __forceinline__ uint32_t swap_pair(uint32_t x) {
+  constexpr int kSwap1 = 1 | (0 << 2) | (3 << 4) | (2 << 6);  // quad_perm: lane ^ 1
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kSwap1, 0xf, 0xf, false);
 }
 
-// ---- paged 5-D layout: one wavefront per (token, head) ------------------------
+template <class KT, class CT>
+__device__ __forceinline__ typename Vec8<CT>::type load_v_task(const typename Elem<KT>::storage* src, int64_t stride,
+                                                               bool odd, const Fp8Scale& s) {
+  if constexpr (std::is_same<CT, FP8>::value) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const Pair<KT> w = load_pair<KT>(src + e * stride);
+      x[e] = w.a;
+      x[4 + e] = w.b;
+    }
+    const uint32_t d0 = fp8_encode4_scaled(x, s), d1 = fp8_encode4_scaled(x + 4, s);
+    const uint32_t s0 = swap_pair(d0), s1 = swap_pair(d1);
+    return odd ? make_uint2(s1, d1) : make_uint2(d0, s0);
+  } else {
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (std::is_same<KT, CT>::value) {
+        w[e] = *reinterpret_cast<const uint32_t*>(src + e * stride);
+      } else {
+        const Pair<KT> x = load_pair<KT>(src + e * stride);
+        w[e] = pack2(from_f32<CT>(x.a), from_f32<CT>(x.b));
+      }
+    }
+    // Low halves: dimension d0 of tokens 0 1 | 2 3; high halves: d0 + 1.
+    const uint2 d0 = make_uint2(__builtin_amdgcn_perm(w[1], w[0], 0x05040100u),
+                                __builtin_amdgcn_perm(w[3], w[2], 0x05040100u));
+    const uint2 d1 = make_uint2(__builtin_amdgcn_perm(w[1], w[0], 0x07060302u),
+                                __builtin_amdgcn_perm(w[3], w[2], 0x07060302u));
+    const uint2 s0 = make_uint2(swap_pair(d0.x), swap_pair(d0.y)), s1 = make_uint2(swap_pair(d1.x), swap_pair(d1.y));
+    return odd ? make_uint4(s1.x, s1.y, d1.x, d1.y) : make_uint4(d0.x, d0.y, s0.x, s0.y);
+  }
+}
+
+template <class KT, class CT, int BS>
+__global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int hg, int head_groups, int parts) {
+  using KS = typename Elem<KT>::storage;
+  using CS = typename Elem<CT>::storage;
+  constexpr bool F8 = std::is_same<CT, FP8>::value;
+  constexpr int X = 16 / Elem<CT>::kBytes;  // elements per 16-byte K chunk
+  const int tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wg = blockIdx.x / (uint32_t)parts;
+  const int part = (int)(blockIdx.x - wg * (uint32_t)parts);
+  const int64_t window = wg / (uint32_t)head_groups;
+  const int h0 = (int)(wg - (uint32_t)window * (uint32_t)head_groups) * hg;
+  const int first = part * 256 + tid, step = parts * 256;  // this thread's tasks
+  const int nh = min(hg, p.num_heads - h0);
+  const int D = p.head_size;
+  const Fp8Scale ks{p.k_scale, p.k_inv, p.fast_div != 0}, vs{p.v_scale, p.v_inv, p.fast_div != 0};
+  const KS* key = static_cast<const KS*>(p.key) + (int64_t)h0 * D;
+  const KS* val = static_cast<const KS*>(p.value) + (int64_t)h0 * D;
+  CS* kc = static_cast<CS*>(p.key_cache);
+  CS* vc = static_cast<CS*>(p.value_cache);
+
+  int64_t prev, run;
+  int lane_slot;
+  rac_window_runs<BS>(p, window, lane, prev, run, lane_slot);
+
+  if (run >= 0) {
+    const int units = D * (BS / 8);  // tasks per head
+    const int64_t blk = p.slot_mapping[run] / BS;
+    const KS* k0 = key + run * p.key_stride;
+    const KS* v0 = val + run * p.value_stride;
+    const int64_t region0 = (blk * p.num_heads + h0) * (int64_t)D * BS;
+    for (int i = first; i < nh * units; i += step) {
+      const int h = nh == 1 ? 0 : i / units;
+      const int u = i - h * units;
+      const int64_t region = region0 + (int64_t)h * D * BS;
+      // K: eight dimensions of one token.
+      int t, d;
+      if constexpr (F8) {
+        t = (u >> 1) % BS;
+        d = (u >> 1) / BS * 16 + (u & 1) * 8;
+      } else {
+        t = u % BS;
+        d = u / BS * 8;
+      }
+      const auto kv = load8<KT, CT>(k0 + t * p.key_stride + h * D + d, ks);
+      // V: dimensions 2 pair, 2 pair + 1 of tokens 4 quad .. +3.
+      const int quad = u % (BS / 4), pair = u / (BS / 4);
+      const auto vv = load_v_task<KT, CT>(v0 + (int64_t)(4 * quad) * p.value_stride + h * D + 2 * pair,
+                                          p.value_stride, (quad & 1) != 0, vs);
+      store8<true>(kc + region + 8 * u, kv);
+      store8<true>(vc + region + (2 * pair + (quad & 1)) * BS + 8 * (quad >> 1), vv);
+    }
+  }
+
+  // The window's other tokens.
+  const int64_t w0 = window * BS;
+  const int64_t s0 = prev >= 0 ? prev + BS : w0;  // prev + BS > w0
+  const int64_t s1 = run >= 0 ? run : min(w0 + BS, p.num_tokens);
+  if (s0 >= s1) return;
+  const int lane0 = (int)(s0 - w0) + BS;  // the lane that holds token s0's slot
+  if constexpr (F8) {
+    // Eight elements of a token's K and V per thread: the encoder works on
+    // groups of four, and one V element per lane (as below) took an
+    // 8192-token prefill of ragged prompts from 15.3 to 18.5 us.  (A
+    // wavefront's trips are the same in every lane: the slots come from other
+    // lanes.)
+    const int per = nh * D / 8, total = (int)(s1 - s0) * per;
+    for (int i = first; i - lane < total; i += step) {
+      const int j = i / per, c = i - j * per;
+      const int64_t tok = s0 + j;
+      const int32_t slot = __shfl(lane_slot, (lane0 + j) & 63);
+      if (i >= total || slot < 0 || (int64_t)slot >= p.num_slots) continue;
+      const int h = nh == 1 ? 0 : 8 * c / D;
+      const int d = 8 * c - h * D;
+      const uint2 kv = load8<KT, CT>(key + tok * p.key_stride + 8 * c, ks);
+      const uint2 vv = load8<KT, CT>(val + tok * p.value_stride + 8 * c, vs);
+      const int64_t region = ((int64_t)(slot / BS) * p.num_heads + h0 + h) * (int64_t)D * BS;
+      store8<false>(kc + region + ((int64_t)(d / X) * BS + slot % BS) * X + d % X, kv);
+      CS* vd = vc + region + d * BS + slot % BS;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) vd[r * BS] = (uint8_t)((r < 4 ? vv.x : vv.y) >> (8 * (r & 3)));
+    }
+    return;
+  } else {
+    // One (token, head) per wavefront and turn, lanes over the K chunks and over
+    // the dimensions of V, so that a store instruction's accesses to one line
+    // (64 / BS dimensions of the token) leave as one request.  (Eight dimensions
+    // per lane: 2,200 random slots of 32-token blocks 40 us against 30.)  The
+    // loads of U turns are issued together and unconditionally, padding lanes
+    // and turns reading the last valid place.
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int pairs = (int)(s1 - s0) * nh, wstep = parts * 4;
+    auto turns = [&](auto count) {
+      constexpr int U = decltype(count)::value;
+      for (int q0 = part * 4 + wave; q0 < pairs; q0 += U * wstep) {
+        uint4 kv[U];
+        KS v0[U], v1[U];
+        int tok[U], head[U];
+  #pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int q = min(q0 + u * wstep, pairs - 1);
+          tok[u] = nh == 1 ? q : q / nh;
+          head[u] = q - tok[u] * nh;
+          const KS* ksrc = key + (s0 + tok[u]) * p.key_stride + head[u] * D;
+          const KS* vsrc = val + (s0 + tok[u]) * p.value_stride + head[u] * D;
+          kv[u] = load8<KT, CT>(ksrc + 8 * min(lane, D / 8 - 1), ks);
+          v0[u] = vsrc[min(lane, D - 1)];
+          v1[u] = vsrc[min(lane + 64, D - 1)];
+        }
+  #pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int32_t slot = __builtin_amdgcn_readlane(lane_slot, lane0 + tok[u]);
+          if (q0 + u * wstep >= pairs || slot < 0 || (int64_t)slot >= p.num_slots) continue;
+          const int64_t region = ((int64_t)(slot / BS) * p.num_heads + h0 + head[u]) * (int64_t)D * BS;
+          CS* kd = kc + region + (slot % BS) * X;
+          CS* vd = vc + region + slot % BS;
+          auto put_k = [&](int c, uint4 x) {
+            CS* to = kd + (int64_t)c * BS * X;
+            if (p.stream_k)
+              store8<true>(to, x);
+            else
+              store8<false>(to, x);
+          };
+          auto put_v = [&](int d, KS x) { vd[(int64_t)d * BS] = convert_elem<KT, CT>(x); };
+          if (lane < D / 8) put_k(lane, kv[u]);
+          if (lane < D) put_v(lane, v0[u]);
+          if (lane + 64 < D) put_v(lane + 64, v1[u]);
+          const KS* ksrc = key + (s0 + tok[u]) * p.key_stride + head[u] * D;
+          const KS* vsrc = val + (s0 + tok[u]) * p.value_stride + head[u] * D;
+          for (int c = lane + 64; c < D / 8; c += 64) put_k(c, load8<KT, CT>(ksrc + 8 * c, ks));
+          for (int d = lane + 128; d < D; d += 64) put_v(d, vsrc[d]);
+        }
+      }
+    };
+    if (pairs <= wstep)
+      turns(std::integral_constant<int, 1>{});
+    else
+      turns(std::integral_constant<int, 4>{});
+  }
+}
+
+// ---- paged 5-D layout, float32 caches, unaligned sources and other block sizes:
+// one wavefront per (token, head) ------------------------------------------------
 template <class KT, class CT, bool ALIGNED>
 __global__ __launch_bounds__(256) void rac_paged5d_kernel(RacParams p) {
   using KS = typename Elem<KT>::storage;
@@ -148,16 +401,6 @@ __global__ __launch_bounds__(256) void rac_paged5d_kernel(RacParams p) {
   if (slot < 0 || (int64_t)slot >= p.num_slots) return;
   const int64_t blk = slot / p.block_size;
   const int off = slot - (int)blk * p.block_size;
-  if constexpr (ALIGNED && Elem<CT>::kBytes == 2) {
-    const int bs = p.block_size;
-    // (Head sizes that are multiples of 8: whole 16-byte units per slice.)
-    if ((bs == 8 || bs == 16 || bs == 32) && p.head_size % 8 == 0 && rac_whole_block(p, tok, slot, off, lane)) {
-      if (bs == 8) rac_run_slice<KT, CT, 8>(p, tok - off, off, head, blk, lane);
-      else if (bs == 16) rac_run_slice<KT, CT, 16>(p, tok - off, off, head, blk, lane);
-      else rac_run_slice<KT, CT, 32>(p, tok - off, off, head, blk, lane);
-      return;
-    }
-  }
   const int D = p.head_size;
   const KS* ksrc = static_cast<const KS*>(p.key) + tok * p.key_stride + (int64_t)head * D;
   const KS* vsrc = static_cast<const KS*>(p.value) + tok * p.value_stride + (int64_t)head * D;
@@ -165,14 +408,9 @@ __global__ __launch_bounds__(256) void rac_paged5d_kernel(RacParams p) {
   CS* kdst = static_cast<CS*>(p.key_cache) + region;    // [D/X][bs][X]
   CS* vdst = static_cast<CS*>(p.value_cache) + region;  // [D][bs]
   const int nchunk = D / X;
-  // K chunks of a large call are stored nontemporally (p.stream_k): a
-  // token's 16-byte chunks sit bs*16 bytes apart, one per line, and a call
-  // writing more K than one XCD's L2 holds (4 MiB) has its lines evicted
-  // before a later token fills their neighbours.  Measured on MI355X at
-  // 4096 random slots (8 MiB of K): 76.4 -> 65.0 us.  A small call keeps
-  // default stores (the reference's append of 8 tokens, rewritten back to
-  // back: 2.45 us default, 3.1 us nontemporal).  V's 2-byte stores keep
-  // default stores: the L2 combines the tokens of a block into lines.
+  // K chunks of a large call are stored nontemporally, as in the window kernel
+  // (a small call keeps default stores: 8 tokens, rewritten back to back, 2.45
+  // us default, 3.1 us nontemporal).
   if (ALIGNED && p.stream_k) {
     for (int c = lane; c < nchunk; c += 64)
       __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, load_vec16<KT, CT>(ksrc + c * X)),
@@ -283,40 +521,8 @@ __global__ __launch_bounds__(64 * kRacWaves) void rac_token_major_wave_kernel(Ra
   }
 }
 
-// ---- FP8 caches -------------------------------------------------------------------
-// E4M3 codes of x / scale (pkv_fp8.h).  Token-major: one wavefront per
-// token, each lane turning 8 source elements into 8 code bytes per step of
-// the K row and of the V row.  Paged 5-D (x = 16): one wavefront per
-// (token, head), K as 16-byte chunks, V as single bytes (token-minor layout).
-__device__ __forceinline__ float fp8_scaled(float x, float scale, float inv, bool pow2) {
-  return pow2 ? x * inv : __fdiv_rn(x, scale);
-}
-
-template <class KT>
-__device__ __forceinline__ uint2 encode8(const typename Elem<KT>::storage* __restrict__ src, float scale, float inv,
-                                         bool pow2) {
-  float v[8];
-  if constexpr (std::is_same<KT, F32>::value) {
-    const float4 a = reinterpret_cast<const float4*>(src)[0], b = reinterpret_cast<const float4*>(src)[1];
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-  } else {
-    const uint4 w = *reinterpret_cast<const uint4*>(src);
-    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = to_f32<KT>((uint16_t)(u[i] & 0xffffu));
-      v[2 * i + 1] = to_f32<KT>((uint16_t)(u[i] >> 16));
-    }
-  }
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lo |= fp8_e4m3_encode(fp8_scaled(v[i], scale, inv, pow2)) << (8 * i);
-    hi |= fp8_e4m3_encode(fp8_scaled(v[4 + i], scale, inv, pow2)) << (8 * i);
-  }
-  return make_uint2(lo, hi);
-}
-
+// ---- FP8 caches, token-major: one wavefront per token, each lane turning 8
+// source elements into 8 code bytes per step of the K row and of the V row. ------
 template <class KT>
 __global__ __launch_bounds__(256) void rac_fp8_token_major_kernel(RacParams p) {
   using KS = typename Elem<KT>::storage;
@@ -327,14 +533,14 @@ __global__ __launch_bounds__(256) void rac_fp8_token_major_kernel(RacParams p) {
   if (slot < 0 || (int64_t)slot >= p.num_slots) return;
   const int row = p.num_heads * p.head_size;  // a multiple of 8
   const int n8 = row / 8;
-  const bool pow2 = p.scales_pow2 != 0;
+  const Fp8Scale ks{p.k_scale, p.k_inv, p.fast_div != 0}, vs{p.v_scale, p.v_inv, p.fast_div != 0};
   const KS* ksrc = static_cast<const KS*>(p.key) + tok * p.key_stride;
   const KS* vsrc = static_cast<const KS*>(p.value) + tok * p.value_stride;
   uint8_t* kdst = static_cast<uint8_t*>(p.key_cache) + (int64_t)slot * row;
   uint8_t* vdst = static_cast<uint8_t*>(p.value_cache) + (int64_t)slot * row;
   for (int i = lane; i < n8; i += 64) {
-    const uint2 k = encode8<KT>(ksrc + 8 * i, p.k_scale, p.k_inv, pow2);
-    const uint2 v = encode8<KT>(vsrc + 8 * i, p.v_scale, p.v_inv, pow2);
+    const uint2 k = encode8<KT>(ksrc + 8 * i, ks);
+    const uint2 v = encode8<KT>(vsrc + 8 * i, vs);
     __builtin_nontemporal_store(k.x, reinterpret_cast<uint32_t*>(kdst + 8 * i));
     __builtin_nontemporal_store(k.y, reinterpret_cast<uint32_t*>(kdst + 8 * i) + 1);
     __builtin_nontemporal_store(v.x, reinterpret_cast<uint32_t*>(vdst + 8 * i));
@@ -342,45 +548,8 @@ __global__ __launch_bounds__(256) void rac_fp8_token_major_kernel(RacParams p) {
   }
 }
 
-// Whole-block runs over FP8 caches (block sizes 16 and 32): as
-// rac_run_slice, with 16-byte units of 16 codes -- K unit u = c*bs + t
-// (dimensions 16c .. 16c+15 of token t), V unit u = d*bs/16 + g (tokens
-// 16g .. 16g+15 of dimension d); D/16 units (D bytes) per wavefront and
-// region.  Each lane encodes two neighbouring codes of the slice, so one
-// store instruction writes D/64 x 128 contiguous bytes and the encodes
-// spread over the whole wavefront.
-template <class KT, int BS>
-__device__ __forceinline__ void rac_fp8_run_slice(const RacParams& p, int64_t first, int off, int head, int64_t blk,
-                                                  int lane) {
-  using KS = typename Elem<KT>::storage;
-  static_assert(BS % 16 == 0, "16-byte units of 16 codes");
-  const int D = p.head_size;
-  const int per = D / 16;
-  const bool pow2 = p.scales_pow2 != 0;
-  const int64_t region = (blk * p.num_heads + head) * (int64_t)D * BS;
-  const int64_t slice = region + (int64_t)off * per * 16;
-  const int64_t hoff = (int64_t)head * D;
-  const KS* key = static_cast<const KS*>(p.key);
-  const KS* val = static_cast<const KS*>(p.value);
-  for (int i = 2 * lane; i < D; i += 128) {
-    const int u = off * per + i / 16, b = i % 16;
-    // K: dimensions 16c + b, +1 of token t.
-    const int c = u / BS, t = u % BS;
-    const KS* ks = key + (first + t) * p.key_stride + hoff + 16 * c + b;
-    const uint32_t k0 = fp8_e4m3_encode(fp8_scaled(to_f32<KT>(ks[0]), p.k_scale, p.k_inv, pow2));
-    const uint32_t k1 = fp8_e4m3_encode(fp8_scaled(to_f32<KT>(ks[1]), p.k_scale, p.k_inv, pow2));
-    // V: tokens 16g + b, +1 of dimension d.
-    const int d = u / (BS / 16), g = u % (BS / 16);
-    const KS* vs = val + (first + 16 * g + b) * p.value_stride + hoff + d;
-    const uint32_t v0 = fp8_e4m3_encode(fp8_scaled(to_f32<KT>(vs[0]), p.v_scale, p.v_inv, pow2));
-    const uint32_t v1 = fp8_e4m3_encode(fp8_scaled(to_f32<KT>(vs[p.value_stride]), p.v_scale, p.v_inv, pow2));
-    __builtin_nontemporal_store((uint16_t)(k0 | (k1 << 8)),
-                                reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(p.key_cache) + slice + i));
-    __builtin_nontemporal_store((uint16_t)(v0 | (v1 << 8)),
-                                reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(p.value_cache) + slice + i));
-  }
-}
-
+// ---- FP8 caches, paged 5-D layout, other block sizes: one wavefront per (token,
+// head), K as 8-byte halves of the 16-byte chunks, V as single bytes. -------------
 template <class KT>
 __global__ __launch_bounds__(256) void rac_fp8_paged5d_kernel(RacParams p) {
   using KS = typename Elem<KT>::storage;
@@ -394,29 +563,54 @@ __global__ __launch_bounds__(256) void rac_fp8_paged5d_kernel(RacParams p) {
   const int64_t blk = slot / p.block_size;
   const int off = slot - (int)blk * p.block_size;
   const int D = p.head_size;  // a multiple of 16
-  if ((p.block_size == 16 || p.block_size == 32) && rac_whole_block(p, tok, slot, off, lane)) {
-    if (p.block_size == 16) rac_fp8_run_slice<KT, 16>(p, tok - off, off, head, blk, lane);
-    else rac_fp8_run_slice<KT, 32>(p, tok - off, off, head, blk, lane);
-    return;
-  }
-  const bool pow2 = p.scales_pow2 != 0;
+  const Fp8Scale ks{p.k_scale, p.k_inv, p.fast_div != 0}, vs{p.v_scale, p.v_inv, p.fast_div != 0};
   const KS* ksrc = static_cast<const KS*>(p.key) + tok * p.key_stride + (int64_t)head * D;
   const KS* vsrc = static_cast<const KS*>(p.value) + tok * p.value_stride + (int64_t)head * D;
   const int64_t region = ((int64_t)blk * p.num_heads + head) * (int64_t)D * p.block_size;
   uint8_t* kdst = static_cast<uint8_t*>(p.key_cache) + region;    // [D/16][bs][16]
   uint8_t* vdst = static_cast<uint8_t*>(p.value_cache) + region;  // [D][bs]
   for (int c = lane; c < D / 8; c += 64) {  // 8-element halves of the 16-byte chunks
-    const uint2 k = encode8<KT>(ksrc + 8 * c, p.k_scale, p.k_inv, pow2);
+    const uint2 k = encode8<KT>(ksrc + 8 * c, ks);
     *reinterpret_cast<uint2*>(kdst + ((int64_t)(c >> 1) * p.block_size + off) * 16 + (c & 1) * 8) = k;
   }
   for (int d = lane; d < D; d += 64)
     vdst[(int64_t)d * p.block_size + off] =
-        (uint8_t)fp8_e4m3_encode(fp8_scaled(to_f32<KT>(vsrc[d]), p.v_scale, p.v_inv, pow2));
+        (uint8_t)fp8_e4m3_encode(__fdiv_rn(to_f32<KT>(vsrc[d]), vs.scale));
+}
+
+// Paged 5-D caches of 16-bit and FP8 elements with blocks of 8, 16 or 32
+// tokens: the window kernel at every number of tokens (*ok: it took the call).
+// Heads per window and 256 threads: as many as give every thread a run task.
+// A small call splits each window over as many workgroups as give every
+// scattered token (16-bit caches: (token, head)) a turn of its own.
+constexpr int64_t kWindowSplitBelow = 512;  // workgroups: two per CU
+template <class KT, class CT>
+static hipError_t launch_paged_window(const RacParams& p, hipStream_t stream, bool* ok) {
+  const int bs = p.block_size;
+  *ok = (bs == 8 || bs == 16 || bs == 32) && p.head_size % 8 == 0;
+  if (!*ok) return hipSuccess;
+  const int units = p.head_size * (bs / 8);
+  const int hg = std::min(p.num_heads, (256 + units - 1) / units);
+  const int groups = (p.num_heads + hg - 1) / hg;
+  const int64_t wgs = (p.num_tokens + bs - 1) / bs * groups;
+  const int split = std::max(1, std::is_same<CT, FP8>::value ? bs * hg * p.head_size / 2048 : bs * hg / 4);
+  const int parts = wgs < kWindowSplitBelow ? split : 1;
+  const dim3 grid((unsigned)(wgs * parts)), block(256);
+  if (bs == 8)
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, 8>), grid, block, 0, stream, p, hg, groups, parts);
+  else if (bs == 16)
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, 16>), grid, block, 0, stream, p, hg, groups, parts);
+  else
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, 32>), grid, block, 0, stream, p, hg, groups, parts);
+  return hipGetLastError();
 }
 
 template <class KT>
 static hipError_t launch_rac_fp8(const RacParams& p, hipStream_t stream) {
   if (p.layout == 0) {
+    bool ok;
+    const hipError_t e = launch_paged_window<KT, FP8>(p, stream, &ok);
+    if (ok) return e;
     const int64_t waves = p.num_tokens * p.num_heads;
     hipLaunchKernelGGL((rac_fp8_paged5d_kernel<KT>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, p);
   } else {
@@ -430,6 +624,13 @@ static hipError_t launch_rac_fp8(const RacParams& p, hipStream_t stream) {
 template <class KT, class CT>
 static hipError_t launch_rac_typed(const RacParams& p, bool aligned, hipStream_t stream) {
   if (p.layout == 0) {
+    if constexpr (Elem<CT>::kBytes == 2) {
+      if (aligned) {
+        bool ok;
+        const hipError_t e = launch_paged_window<KT, CT>(p, stream, &ok);
+        if (ok) return e;
+      }
+    }
     const int64_t waves = p.num_tokens * p.num_heads;
     const dim3 grid((unsigned)((waves + 3) / 4));
     if (aligned)

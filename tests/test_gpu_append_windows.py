@@ -1,0 +1,92 @@
+"""GPU parity of the paged append's window kernel, bit-exact over whole caches:
+whole-block runs at every offset of a window, runs broken at their first, a
+middle and their last token, the cache's last block, padding and slots past the
+cache, head sizes whose run tasks do not fill a workgroup, and FP8 codes whose
+quotients are ties, subnormals, overflows and zeros, at scales with and without
+an exact reciprocal and beyond the range of the corrected division."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import pagedkv_oracle as orc
+from pkv_torch import to_index, to_numpy, to_torch
+from sglang_mlx_amd import kernels
+
+pytestmark = pytest.mark.gpu
+
+FP8 = "fp8_e4m3"
+
+
+def window_slots(bs, nb, seed):
+    """Slots of one call: whole blocks separated by 1 .. bs-1 other tokens, so
+    that runs start at every offset of a window."""
+    rng = np.random.default_rng(seed)
+    free = [b for b in rng.permutation(nb - 1).tolist()]
+    whole = lambda b: list(range(b * bs, (b + 1) * bs))  # noqa: E731
+    out = []
+    for lead in range(bs):
+        out += whole(free.pop())
+        single = free.pop()
+        out += [single * bs + t for t in rng.permutation(bs)[:lead].tolist()]  # scattered in one block
+    out += whole(nb - 1)  # the cache's last block
+    broken = whole(free.pop())
+    out += broken[1:]  # starts at offset 1
+    hole = whole(free.pop())
+    hole[bs // 2] = -1
+    out += hole + whole(free.pop())
+    late = whole(free.pop())
+    late[-1] = nb * bs + 5  # past the cache
+    out += late + whole(free.pop())[:-1]  # ends a token short, at the batch's end
+    return np.array(out, dtype=np.int32)
+
+
+def check(bs, H, D, kv_dtype, cache_dtype, seed, scales=(1.0, 1.0), values=None):
+    x = 16 if cache_dtype == FP8 else 8
+    nb = 3 * bs + 16
+    slots = window_slots(bs, nb, seed)
+    rng = np.random.default_rng(seed)
+    N = len(slots)
+    if values is None:
+        raw = rng.standard_normal((2, N, H, D), dtype=np.float32)
+    else:
+        raw = rng.choice(values, size=(2, N, H, D)).astype(np.float32)
+    key, value = (raw if kv_dtype == "float32" else orc.to_storage(raw, kv_dtype))
+    top, word = (256, np.uint8) if cache_dtype == FP8 else (65536, np.uint16)
+    kc0 = rng.integers(0, top, size=(nb, H, D // x, bs, x)).astype(word)
+    vc0 = rng.integers(0, top, size=(nb, H, D, bs)).astype(word)
+    kc, vc = to_torch(kc0, cache_dtype), to_torch(vc0, cache_dtype)
+    kernels.reshape_and_cache(to_torch(key, kv_dtype), to_torch(value, kv_dtype), kc, vc, to_index(slots),
+                              k_scale=scales[0], v_scale=scales[1])
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        # (Slots past the cache are skipped, as padding is.)
+        rk, rv = orc.reshape_and_cache_paged5d(key, value, kc0, vc0, np.where(slots < nb * bs, slots, -1), kv_dtype,
+                                               cache_dtype, *scales)
+    np.testing.assert_array_equal(to_numpy(kc), rk)
+    np.testing.assert_array_equal(to_numpy(vc), rv)
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("H,D", [(1, 32), (3, 80), (2, 120), (5, 128), (2, 256)])
+@pytest.mark.parametrize("pair", [("bfloat16", "bfloat16"), ("float32", "float16")])
+def test_16_bit(bs, H, D, pair):
+    check(bs, H, D, *pair, seed=bs + D)
+
+
+# Quotients times the scale: ties of every exponent, subnormals and their
+# half-way points, the edges 2^-9, 2^-6, 240, 248, 256 and 2^14, zeros.
+QUOTIENTS = np.array([s * v for s in (1.0, -1.0)
+                      for v in ([0.0, 1e-30, 2.0 ** -10, 2.0 ** -9 * 0.999, 240.0, 247.9, 248.0, 255.0, 256.0, 300.0,
+                                 16383.0, 16384.0, 1e30, np.inf]
+                                + [(1 + m / 16) * 2.0 ** e for m in range(16) for e in range(-11, 8)])])
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("H,D", [(1, 32), (3, 80), (3, 128)])
+@pytest.mark.parametrize("kv_dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("scales", [(0.05, 0.02), (-0.7, 1.0 / 3.0), (0.125, 2.0), (1e-25, 2.0 ** 61)])
+def test_fp8(bs, H, D, kv_dtype, scales):
+    with np.errstate(over="ignore"):
+        values = (QUOTIENTS * np.float32(scales[0])).astype(np.float32)
+    check(bs, H, D, kv_dtype, FP8, seed=bs + D, scales=scales, values=values)
