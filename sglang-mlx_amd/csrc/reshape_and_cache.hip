@@ -91,7 +91,7 @@ __device__ __forceinline__ uint2 encode8(const typename Elem<KT>::storage* __res
 }
 
 // ---- paged 5-D layout, windows of one block's tokens ------------------------------
-// One workgroup (or `parts` that share its tasks) per (window of BS
+// One workgroup (SPLIT: several that share its tasks) per (window of BS
 // consecutive batch tokens, group of `hg` heads), for block sizes 8, 16 and
 // 32.  When BS consecutive batch tokens write slots blk*BS .. blk*BS + BS-1 in
 // order (a prefill writing whole blocks, a "run"), the (block, head) regions
@@ -245,17 +245,16 @@ __device__ __forceinline__ typename Vec8<CT>::type load_v_task(const typename El
   }
 }
 
-template <class KT, class CT, int BS>
-__global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int hg, int head_groups, int parts) {
+template <class KT, class CT, int BS, bool SPLIT>
+__global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int hg, int head_groups) {
   using KS = typename Elem<KT>::storage;
   using CS = typename Elem<CT>::storage;
   constexpr bool F8 = std::is_same<CT, FP8>::value;
   constexpr int X = 16 / Elem<CT>::kBytes;  // elements per 16-byte K chunk
   const int tid = threadIdx.x, lane = tid & 63;
-  const uint32_t wg = blockIdx.x / (uint32_t)parts;
-  const int part = (int)(blockIdx.x - wg * (uint32_t)parts);
-  const int64_t window = wg / (uint32_t)head_groups;
-  const int h0 = (int)(wg - (uint32_t)window * (uint32_t)head_groups) * hg;
+  const int part = SPLIT ? (int)blockIdx.y : 0, parts = SPLIT ? (int)gridDim.y : 1;
+  const int64_t window = head_groups == 1 ? blockIdx.x : blockIdx.x / (uint32_t)head_groups;
+  const int h0 = (int)(blockIdx.x - (uint32_t)window * (uint32_t)head_groups) * hg;
   const int first = part * 256 + tid, step = parts * 256;  // this thread's tasks
   const int nh = min(hg, p.num_heads - h0);
   const int D = p.head_size;
@@ -264,6 +263,23 @@ __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int 
   const KS* val = static_cast<const KS*>(p.value) + (int64_t)h0 * D;
   CS* kc = static_cast<CS*>(p.key_cache);
   CS* vc = static_cast<CS*>(p.value_cache);
+
+  // SPLIT, 16-bit caches: the wavefront's own (token, head) of the window, whose
+  // loads go out before the slots are known.
+  constexpr bool kOwn = SPLIT && !F8;
+  const int64_t w0 = window * BS;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint4 own_k = make_uint4(0, 0, 0, 0);
+  KS own_v0 = 0, own_v1 = 0;
+  const int own_tok = part * 4 + wave;  // (one head per workgroup)
+  if constexpr (kOwn) {
+    const int64_t tok = min(w0 + own_tok, p.num_tokens - 1);
+    const KS* ksrc = key + tok * p.key_stride;
+    const KS* vsrc = val + tok * p.value_stride;
+    own_k = load8<KT, CT>(ksrc + 8 * min(lane, D / 8 - 1), ks);
+    own_v0 = vsrc[min(lane, D - 1)];
+    own_v1 = vsrc[min(lane + 64, D - 1)];
+  }
 
   int64_t prev, run;
   int lane_slot;
@@ -299,7 +315,6 @@ __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int 
   }
 
   // The window's other tokens.
-  const int64_t w0 = window * BS;
   const int64_t s0 = prev >= 0 ? prev + BS : w0;  // prev + BS > w0
   const int64_t s1 = run >= 0 ? run : min(w0 + BS, p.num_tokens);
   if (s0 >= s1) return;
@@ -333,55 +348,54 @@ __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int 
     // (64 / BS dimensions of the token) leave as one request.  (Eight dimensions
     // per lane: 2,200 random slots of 32-token blocks 40 us against 30.)  The
     // loads of U turns are issued together and unconditionally, padding lanes
-    // and turns reading the last valid place.
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int pairs = (int)(s1 - s0) * nh, wstep = parts * 4;
-    auto turns = [&](auto count) {
-      constexpr int U = decltype(count)::value;
-      for (int q0 = part * 4 + wave; q0 < pairs; q0 += U * wstep) {
+    // and turns reading the last valid place.  SPLIT: one turn per wavefront.
+    auto put = [&](int tok, int head, uint4 kx, KS v0, KS v1) {  // tok: counted from w0
+      const int32_t slot = __builtin_amdgcn_readlane(lane_slot, BS + tok);
+      if (slot < 0 || (int64_t)slot >= p.num_slots) return;
+      const int64_t region = ((int64_t)(slot / BS) * p.num_heads + h0 + head) * (int64_t)D * BS;
+      CS* kd = kc + region + (slot % BS) * X;
+      CS* vd = vc + region + slot % BS;
+      auto put_k = [&](int c, uint4 x) {
+        CS* to = kd + (int64_t)c * BS * X;
+        if (p.stream_k)
+          store8<true>(to, x);
+        else
+          store8<false>(to, x);
+      };
+      auto put_v = [&](int d, KS x) { vd[(int64_t)d * BS] = convert_elem<KT, CT>(x); };
+      if (lane < D / 8) put_k(lane, kx);
+      if (lane < D) put_v(lane, v0);
+      if (lane + 64 < D) put_v(lane + 64, v1);
+      const KS* ksrc = key + (w0 + tok) * p.key_stride + head * D;
+      const KS* vsrc = val + (w0 + tok) * p.value_stride + head * D;
+      for (int c = lane + 64; c < D / 8; c += 64) put_k(c, load8<KT, CT>(ksrc + 8 * c, ks));
+      for (int d = lane + 128; d < D; d += 64) put_v(d, vsrc[d]);
+    };
+    if constexpr (kOwn) {
+      if (own_tok >= s0 - w0 && own_tok < s1 - w0) put(own_tok, 0, own_k, own_v0, own_v1);
+    } else {
+      constexpr int U = 4;
+      const int pairs = (int)(s1 - s0) * nh;
+      for (int q0 = wave; q0 < pairs; q0 += 4 * U) {
         uint4 kv[U];
         KS v0[U], v1[U];
         int tok[U], head[U];
-  #pragma unroll
+#pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int q = min(q0 + u * wstep, pairs - 1);
-          tok[u] = nh == 1 ? q : q / nh;
-          head[u] = q - tok[u] * nh;
-          const KS* ksrc = key + (s0 + tok[u]) * p.key_stride + head[u] * D;
-          const KS* vsrc = val + (s0 + tok[u]) * p.value_stride + head[u] * D;
+          const int q = min(q0 + 4 * u, pairs - 1);
+          tok[u] = (int)(s0 - w0) + (nh == 1 ? q : q / nh);
+          head[u] = q - (tok[u] - (int)(s0 - w0)) * nh;
+          const KS* ksrc = key + (w0 + tok[u]) * p.key_stride + head[u] * D;
+          const KS* vsrc = val + (w0 + tok[u]) * p.value_stride + head[u] * D;
           kv[u] = load8<KT, CT>(ksrc + 8 * min(lane, D / 8 - 1), ks);
           v0[u] = vsrc[min(lane, D - 1)];
           v1[u] = vsrc[min(lane + 64, D - 1)];
         }
-  #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int32_t slot = __builtin_amdgcn_readlane(lane_slot, lane0 + tok[u]);
-          if (q0 + u * wstep >= pairs || slot < 0 || (int64_t)slot >= p.num_slots) continue;
-          const int64_t region = ((int64_t)(slot / BS) * p.num_heads + h0 + head[u]) * (int64_t)D * BS;
-          CS* kd = kc + region + (slot % BS) * X;
-          CS* vd = vc + region + slot % BS;
-          auto put_k = [&](int c, uint4 x) {
-            CS* to = kd + (int64_t)c * BS * X;
-            if (p.stream_k)
-              store8<true>(to, x);
-            else
-              store8<false>(to, x);
-          };
-          auto put_v = [&](int d, KS x) { vd[(int64_t)d * BS] = convert_elem<KT, CT>(x); };
-          if (lane < D / 8) put_k(lane, kv[u]);
-          if (lane < D) put_v(lane, v0[u]);
-          if (lane + 64 < D) put_v(lane + 64, v1[u]);
-          const KS* ksrc = key + (s0 + tok[u]) * p.key_stride + head[u] * D;
-          const KS* vsrc = val + (s0 + tok[u]) * p.value_stride + head[u] * D;
-          for (int c = lane + 64; c < D / 8; c += 64) put_k(c, load8<KT, CT>(ksrc + 8 * c, ks));
-          for (int d = lane + 128; d < D; d += 64) put_v(d, vsrc[d]);
-        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (q0 + 4 * u < pairs) put(tok[u], head[u], kv[u], v0[u], v1[u]);
       }
-    };
-    if (pairs <= wstep)
-      turns(std::integral_constant<int, 1>{});
-    else
-      turns(std::integral_constant<int, 4>{});
+    }
   }
 }
 
@@ -581,28 +595,41 @@ __global__ __launch_bounds__(256) void rac_fp8_paged5d_kernel(RacParams p) {
 // Paged 5-D caches of 16-bit and FP8 elements with blocks of 8, 16 or 32
 // tokens: the window kernel at every number of tokens (*ok: it took the call).
 // Heads per window and 256 threads: as many as give every thread a run task.
-// A small call splits each window over as many workgroups as give every
-// scattered token (16-bit caches: (token, head)) a turn of its own.
-constexpr int64_t kWindowSplitBelow = 512;  // workgroups: two per CU
+// A small call takes one head per workgroup and splits each window over as
+// many workgroups as give every token (FP8: eight elements) a wavefront
+// (thread) of its own; the split index is the grid's slower one, so that the
+// parts of a window mostly share an XCD and its L2 combines a block's tokens
+// into lines (902 ragged tokens of 32-token blocks 11.0 -> 5.7 us).  The line:
+// the (token, head) wavefronts that the chip holds at once (32 per CU).
+// (Four heads of one token per workgroup instead of four tokens of one head:
+// 500 scattered windows of 16 5.2 -> 7.4 us.)
+constexpr int64_t kWindowSplitBelow = 8192;
+template <class KT, class CT, int BS>
+static hipError_t launch_window_bs(const RacParams& p, hipStream_t stream) {
+  const int64_t windows = (p.num_tokens + BS - 1) / BS;
+  if (p.num_tokens * p.num_heads < kWindowSplitBelow) {
+    const int parts = std::is_same<CT, FP8>::value ? std::max(1, BS * p.head_size / 2048) : BS / 4;
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, true>),
+                       dim3((unsigned)(windows * p.num_heads), (unsigned)parts), dim3(256), 0, stream, p, 1,
+                       p.num_heads);
+  } else {
+    const int units = p.head_size * (BS / 8);
+    const int hg = std::min(p.num_heads, (256 + units - 1) / units);
+    const int groups = (p.num_heads + hg - 1) / hg;
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, false>), dim3((unsigned)(windows * groups)), dim3(256), 0,
+                       stream, p, hg, groups);
+  }
+  return hipGetLastError();
+}
+
 template <class KT, class CT>
 static hipError_t launch_paged_window(const RacParams& p, hipStream_t stream, bool* ok) {
-  const int bs = p.block_size;
-  *ok = (bs == 8 || bs == 16 || bs == 32) && p.head_size % 8 == 0;
-  if (!*ok) return hipSuccess;
-  const int units = p.head_size * (bs / 8);
-  const int hg = std::min(p.num_heads, (256 + units - 1) / units);
-  const int groups = (p.num_heads + hg - 1) / hg;
-  const int64_t wgs = (p.num_tokens + bs - 1) / bs * groups;
-  const int split = std::max(1, std::is_same<CT, FP8>::value ? bs * hg * p.head_size / 2048 : bs * hg / 4);
-  const int parts = wgs < kWindowSplitBelow ? split : 1;
-  const dim3 grid((unsigned)(wgs * parts)), block(256);
-  if (bs == 8)
-    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, 8>), grid, block, 0, stream, p, hg, groups, parts);
-  else if (bs == 16)
-    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, 16>), grid, block, 0, stream, p, hg, groups, parts);
-  else
-    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, 32>), grid, block, 0, stream, p, hg, groups, parts);
-  return hipGetLastError();
+  *ok = p.head_size % 8 == 0;
+  if (*ok && p.block_size == 8) return launch_window_bs<KT, CT, 8>(p, stream);
+  if (*ok && p.block_size == 16) return launch_window_bs<KT, CT, 16>(p, stream);
+  if (*ok && p.block_size == 32) return launch_window_bs<KT, CT, 32>(p, stream);
+  *ok = false;
+  return hipSuccess;
 }
 
 template <class KT>
