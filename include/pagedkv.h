@@ -123,6 +123,17 @@ size_t pkv_paged_attention_workspace_size(int32_t num_seqs, int32_t num_heads,
                                           int32_t max_seq_len,
                                           int32_t partition_size);
 
+/* Bytes of a workspace that lets pkv_paged_attention take every kernel it has:
+ * at least the above, and room for the piece states of the split kernel, which
+ * balances batches of few, long and uneven contexts over the chip.  With less
+ * (but at least the above) such a batch runs the other kernels, to the same
+ * result within rounding.  Returns 0 where the above does. */
+size_t pkv_paged_attention_full_workspace_size(int32_t num_seqs, int32_t num_heads,
+                                          int32_t num_kv_heads,
+                                          int32_t head_size,
+                                          int32_t max_seq_len,
+                                          int32_t partition_size);
+
 /*
  * Block-table decode attention.
  * Replaces PagedAttentionV1 (mlx_paged_attention.cpp:93-144, :150-213);

@@ -35,6 +35,9 @@
 //   partitions, M = max m_p, w_p = l_p * 2^(m_p - M),
 //   out = sum_p w_p o_p / (sum_p w_p + 1e-6).
 //
+// paged_decode_split_kernel takes their place for batches of few, long and
+// uneven contexts (described there, with the rule in launch_split).
+//
 // The split is invisible in the result: sum_p w_p equals the single-pass
 // softmax denominator, so the merge is an algebraic identity with the
 // reference's single softmax.
@@ -1456,6 +1459,48 @@ __device__ __forceinline__ void store4(typename Elem<QT>::storage* dst, float a,
   }
 }
 
+// ---------------------------------------------------------------------------
+// States that cross workgroups inside one launch (the partition kernel's own
+// merge, and the split kernel's pieces): each workgroup stores its state, then
+// counts it on the row's arrival counter, and the workgroup whose state is the
+// last to arrive merges.  gfx950's L2 caches are per XCD and not coherent
+// with one another for ordinary accesses, so the states are written and read
+// with agent-scope relaxed atomic accesses, which gfx950 issues as ordinary
+// vector loads and stores carrying the SC1 cache-policy bit: each one is
+// coherent at agent scope by itself, with no cache-wide write-back or
+// invalidate.  A writer waits until its stores have completed (s_waitcnt
+// vmcnt(0)) before its relaxed agent-scope atomic add on the counter, so a
+// workgroup that sees the last count can only load states that are already
+// at the coherence point.  The last arrival sets the counter back to zero
+// for the next launch.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void store_agent2(float* p, float a, float b) {
+  const uint64_t v = (uint64_t)__float_as_uint(a) | ((uint64_t)__float_as_uint(b) << 32);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_agent(float* p, float a) {
+  __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __float_as_uint(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_agent2(const float* p) {
+  const uint64_t v =
+      __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+}
+// Waits until this wavefront's vector memory accesses so far have completed;
+// the compiler fences keep every access on its side of the wait.
+__device__ __forceinline__ void wait_stores() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); expcnt and lgkmcnt left at their maxima
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+// Counts one arrival; true for the expected-th, which resets the counter
+// (every arrival of this launch has happened by then).
+__device__ __forceinline__ bool arrive_last(int32_t* counter, int expected) {
+  const bool last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expected - 1;
+  if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return last;
+}
+
 // Merge of the NW wavefronts' states that leaves every wavefront with an
 // equal share of the output: each wavefront moves its state onto its true
 // maximum and stores it in LDS; after one barrier, wavefront w combines
@@ -1465,12 +1510,15 @@ __device__ __forceinline__ void store4(typename Elem<QT>::storage* dst, float a,
 // The weights and sums follow the same order as merge_waves, so the result
 // is the reference's sum(exp(s - max) v) / (sum(exp(s - max)) + 1e-6).
 // hrow: the output row of the lane's column; active: whether the column
-// has one.
-template <class QT, int D, int NW, bool ROWS = false>
+// has one.  state_o / state_ml (STATE, workgroup-uniform): when not null the
+// workgroup holds a piece of its item, and its normalised output and (max,
+// sum) go there instead, row `col` of D (of 2) floats.
+template <class QT, int D, int NW, bool ROWS = false, bool STATE = false>
 __device__ __forceinline__ void merge_store_waves(const DecodeParams& p, WaveAcc<D>& acc,
                                                   float4 (*s_red)[Tile<D>::DT][64], float (*s_m)[16],
                                                   float (*s_l)[16], int wave, int lane, int g, int col, int64_t hrow,
-                                                  bool active) {
+                                                  bool active, float* state_o = nullptr,
+                                                  float* state_ml = nullptr) {
   using QS = typename Elem<QT>::storage;
   constexpr int DT = Tile<D>::DT;
   acc.reduce_max();
@@ -1502,8 +1550,10 @@ __device__ __forceinline__ void merge_store_waves(const DecodeParams& p, WaveAcc
     aw[w] = exp2f(s_m[w][col] - mu);
     L += s_l[w][col] * aw[w];
   }
-  const float inv = p.v_scale / (L + 1e-6f);
+  const bool state = STATE && state_o != nullptr;
+  const float inv = state ? (L > 0.f ? p.v_scale / L : 0.f) : p.v_scale / (L + 1e-6f);
   QS* out = static_cast<QS*>(p.out) + hrow * D;
+  if (state && wave == 0 && g == 0) store_agent2(state_ml + 2 * col, M, L);
   for (int dt = wave; dt < DT; dt += NW) {
     const int d0 = tile_dim<D, ROWS>(dt, g);
     if (D % 16 != 0 && d0 >= D) continue;  // head sizes are multiples of 8
@@ -1520,7 +1570,18 @@ __device__ __forceinline__ void merge_store_waves(const DecodeParams& p, WaveAcc
       o.z += aw[w] * x.z;
       o.w += aw[w] * x.w;
     }
-    if constexpr (RowsWhole<D, ROWS>::value) {
+    if (state) {
+      float* so = state_o + col * D;
+      if constexpr (RowsWhole<D, ROWS>::value) {
+        store_agent(so + out_dim<D, ROWS>(dt, g, 0), o.x * inv);
+        store_agent(so + out_dim<D, ROWS>(dt, g, 1), o.y * inv);
+        store_agent(so + out_dim<D, ROWS>(dt, g, 2), o.z * inv);
+        store_agent(so + out_dim<D, ROWS>(dt, g, 3), o.w * inv);
+      } else {
+        store_agent2(so + d0, o.x * inv, o.y * inv);
+        store_agent2(so + d0 + 2, o.z * inv, o.w * inv);
+      }
+    } else if constexpr (RowsWhole<D, ROWS>::value) {
       out[out_dim<D, ROWS>(dt, g, 0)] = from_f32<QT>(o.x * inv);
       out[out_dim<D, ROWS>(dt, g, 1)] = from_f32<QT>(o.y * inv);
       out[out_dim<D, ROWS>(dt, g, 2)] = from_f32<QT>(o.z * inv);
@@ -1536,45 +1597,6 @@ __device__ __forceinline__ void unit_heads(const DecodeParams& p, int unit, int&
   const int slice = unit - kvh * p.slices;
   h0 = kvh * p.group + slice * 16;
   nh = min(16, p.group - slice * 16);
-}
-
-// ---------------------------------------------------------------------------
-// The partition kernel's own merge.  Partition states cross workgroups inside
-// one launch: each workgroup stores its state, then counts it on its
-// (sequence, unit)'s arrival counter, and the workgroup whose state is the
-// last to arrive merges.  gfx950's L2 caches are per XCD and not coherent
-// with one another for ordinary accesses, so the states are written and read
-// with agent-scope relaxed atomic accesses, which gfx950 issues as ordinary
-// vector loads and stores carrying the SC1 cache-policy bit: each one is
-// coherent at agent scope by itself, with no cache-wide write-back or
-// invalidate.  A writer waits until its stores have completed (s_waitcnt
-// vmcnt(0)) before its relaxed agent-scope atomic add on the counter, so a
-// workgroup that sees the last count can only load states that are already
-// at the coherence point.  The last arrival sets the counter back to zero
-// for the next launch.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void store_agent2(float* p, float a, float b) {
-  const uint64_t v = (uint64_t)__float_as_uint(a) | ((uint64_t)__float_as_uint(b) << 32);
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float2 load_agent2(const float* p) {
-  const uint64_t v =
-      __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
-}
-// Waits until this wavefront's vector memory accesses so far have completed;
-// the compiler fences keep every access on its side of the wait.
-__device__ __forceinline__ void wait_stores() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); expcnt and lgkmcnt left at their maxima
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-// Counts one arrival; true for the expected-th, which resets the counter
-// (every arrival of this launch has happened by then).
-__device__ __forceinline__ bool arrive_last(int32_t* counter, int expected) {
-  const bool last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expected - 1;
-  if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return last;
 }
 
 // Log-sum-exp merge of the `count` partition states (slots 0 .. count-1)
@@ -2017,6 +2039,297 @@ __global__ __launch_bounds__(64 * (Persist<D, BS == 0>::kWaves)) void paged_deco
     merge_store_waves<QT, D, NW, ROWS>(p, acc, s_red[buf], s_m[buf], s_l[buf], wave, lane, g, col,
                                        (int64_t)it.seq * p.num_heads + it.h0 + col, col < it.nh);
     buf ^= 1;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Split kernel: the (sequence, unit) items laid end to end, a span of equal
+// work per workgroup of four wavefronts, as many workgroups as are resident at
+// once.  An item that span boundaries meet inside is computed in pieces; their
+// states meet in the workspace and the workgroup whose piece arrives last
+// merges them.  Every workgroup works the schedule out alike from the context
+// lengths: the host does not know them.
+// ---------------------------------------------------------------------------
+
+// Work is counted in 16-token tiles.  kItemTiles: what starting an item costs
+// (block ids, query, pipeline fill, merge), in tiles.  kMinPiece: the shortest
+// piece a split leaves.  kMinSpan: the least work of a workgroup.
+constexpr int kSplitWaves = 4;
+constexpr int kItemTiles = 16;
+constexpr int kMinPiece = 4;
+constexpr int kMinSpan = 16;
+// Most workgroups per item of the average length.
+constexpr int kMaxPieces = 32;
+// Tokens whose block (row) ids a workgroup holds at a time; longer pieces take
+// several passes.
+constexpr int kSplitPass = 4096, kSplitRowsPass = 2048;
+
+// Tiles of a sequence (0: an empty or over-long context, whose rows are zero).
+__device__ __forceinline__ int seq_tiles(const DecodeParams& p, uint32_t ctx) {
+  return ctx > (uint32_t)p.max_seq_len ? 0 : (int)((ctx + kTile - 1) / kTile);
+}
+
+// s_pref[s]: the sum of (tiles + kItemTiles) over the sequences before s (of
+// one unit each), s_pref[B] the total; returns the span.  Every thread of the
+// workgroup calls it; needs B <= kPersistMaxOrder.
+template <int NT>
+__device__ __forceinline__ int plan_spans(const DecodeParams& p, int32_t* s_pref, int32_t* s_tmp, int tid, int G) {
+  constexpr int NW = NT / 64, PER = kPersistMaxOrder / NT;
+  const int B = p.num_seqs;
+  const int lane = tid & 63, wave = tid >> 6;
+  int v[PER], sum = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int s = tid * PER + k;
+    v[k] = s < B ? seq_tiles(p, (uint32_t)p.context_lens[s]) + kItemTiles : 0;
+    sum += v[k];
+  }
+  int incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o);
+    incl += lane >= o ? y : 0;
+  }
+  if (lane == 63) s_tmp[wave] = incl;
+  __syncthreads();
+  int at = incl - sum;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) at += w < wave ? s_tmp[w] : 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int s = tid * PER + k;
+    if (s <= B) s_pref[s] = at;
+    at += v[k];
+  }
+  if (tid == NT - 1) s_pref[kPersistMaxOrder] = at;
+  __syncthreads();
+  return max((p.units * s_pref[B] + G - 1) / G, kMinSpan);
+}
+
+// A place in the split schedule: tile `off` of item (seq, unit).
+struct SplitPos {
+  int seq, unit, off;
+};
+// Where workgroup w's span begins.  The span's own boundary is moved to an
+// item's start or end where it would leave a piece shorter than kMinPiece.
+__device__ __forceinline__ SplitPos split_pos(const int32_t* s_pref, int B, int units, int span, int w, int lane) {
+  const int x = w * span;
+  if (x >= units * s_pref[B]) return {B, 0, 0};
+  // The last sequence that starts at or before x, in two steps of one lane each.
+  const int stride = (B + 63) >> 6;
+  const int c = min(lane * stride, B);
+  const int hi = __popcll(__ballot(c < B && units * s_pref[c] <= x)) - 1;
+  const int f = hi * stride + lane;
+  const int seq = hi * stride + __popcll(__ballot(lane < stride && f < B && units * s_pref[f] <= x)) - 1;
+  const int len = s_pref[seq + 1] - s_pref[seq], n = len - kItemTiles;
+  const int rem = x - units * s_pref[seq];
+  int unit = rem / len;
+  int off = rem - unit * len - kItemTiles;
+  if (off < kMinPiece) {
+    off = 0;
+  } else if (off > n - kMinPiece) {
+    off = 0;
+    ++unit;
+  }
+  if (unit == units) return {seq + 1, 0, 0};
+  return {seq, unit, off};
+}
+
+// Merges the `pieces` states of a split item's rows and writes them: thread
+// groups of NT / (D/4 * rows) take every groups-th state, four dimensions per
+// thread, and meet in LDS; the states fold in the same order whichever
+// workgroup merges.  The first piece's state lies in slot 2 (w - 1) + 1 and
+// the i-th in slot 2 (w - 1 + i), w being the workgroup whose span starts
+// with the second piece.
+template <class QT, int D, int NT>
+__device__ __forceinline__ void merge_pieces(const DecodeParams& p, int64_t row0, int nh, int pieces, int w,
+                                             float4* s_buf, float2* s_ml, int tid) {
+  using QS = typename Elem<QT>::storage;
+  constexpr int CH = D / 4, U = 4;
+  const int hs = min(16, p.group);  // rows per state slot
+  const int c = tid % CH, t = tid / CH;
+  constexpr int T = NT / CH;        // threads of one chunk: rows x groups
+  const int rows = min(nh, T);      // rows per pass
+  const int groups = T / rows;
+  const int r = t % rows, grp = t / rows;
+  for (int hb = 0; hb < nh; hb += rows) {
+    const bool act = grp < groups && hb + r < nh;
+    const int head = act ? hb + r : 0;
+    float m = -INFINITY, l = 0.f;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i0 = grp; i0 < pieces; i0 += U * groups) {
+      float2 e[U];
+      float4 o[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * groups;
+        e[u] = make_float2(-INFINITY, 0.f);
+        o[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (act && i < pieces) {
+          const int64_t at = (int64_t)(i == 0 ? 2 * w - 1 : 2 * (w - 1 + i)) * hs + head;
+          e[u] = load_agent2(p.split_ml + at * 2);
+          const float2 lo = load_agent2(p.split_o + at * D + 4 * c), hi = load_agent2(p.split_o + at * D + 4 * c + 2);
+          o[u] = make_float4(lo.x, lo.y, hi.x, hi.y);
+        }
+      }
+      float gm = m;
+#pragma unroll
+      for (int u = 0; u < U; ++u) gm = fmaxf(gm, e[u].x);
+      if (gm > m) {
+        const float f = m == -INFINITY ? 0.f : exp2f(m - gm);
+        l *= f, a.x *= f, a.y *= f, a.z *= f, a.w *= f;
+        m = gm;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool use = e[u].x != -INFINITY;
+        const float f = use ? e[u].y * exp2f(e[u].x - m) : 0.f;
+        l += f;
+        a.x += use ? f * o[u].x : 0.f;
+        a.y += use ? f * o[u].y : 0.f;
+        a.z += use ? f * o[u].z : 0.f;
+        a.w += use ? f * o[u].w : 0.f;
+      }
+    }
+    if (groups > 1) {
+      s_buf[tid] = a;
+      if (c == 0) s_ml[t] = make_float2(m, l);
+      __syncthreads();
+      if (act && grp == 0) {
+        for (int q = 1; q < groups; ++q) {
+          const float2 e = s_ml[q * rows + r];
+          const float4 o = s_buf[(q * rows + r) * CH + c];
+          const float gm = fmaxf(m, e.x);
+          const float f0 = m == -INFINITY ? 0.f : exp2f(m - gm), f1 = e.x == -INFINITY ? 0.f : exp2f(e.x - gm);
+          l = l * f0 + e.y * f1;
+          a.x = a.x * f0 + o.x * f1;
+          a.y = a.y * f0 + o.y * f1;
+          a.z = a.z * f0 + o.z * f1;
+          a.w = a.w * f0 + o.w * f1;
+          m = gm;
+        }
+      }
+    }
+    if (act && grp == 0) {
+      const float inv = 1.f / (l + 1e-6f);
+      store4<QT>(static_cast<QS*>(p.out) + (row0 + head) * D + 4 * c, a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+    }
+    __syncthreads();
+  }
+}
+
+// BS = 0: token-row caches (any block size, p.block_size), with each
+// wavefront's row ids in LDS (WaveRows); otherwise the paged layout.
+template <class QT, class CT, int D, int BS>
+__global__ __launch_bounds__(64 * kSplitWaves) void paged_decode_split_kernel(DecodeParams p) {
+  constexpr int NW = kSplitWaves;
+  constexpr int NT = 64 * NW;
+  constexpr int KSTEPS = Tile<D>::KSTEPS;
+  constexpr int DT = Tile<D>::DT;
+  constexpr bool SPLIT_Q = std::is_same<QT, F32>::value;
+  constexpr bool ROWS = BS == 0;
+  constexpr int TBS = ROWS ? kTile : BS;
+  // Tiles per wavefront and pass over a piece (its block or row ids are held
+  // for one pass at a time).
+  constexpr int MAXT = (ROWS ? kSplitRowsPass : kSplitPass) / kTile / NW;
+  using Blocks = std::conditional_t<ROWS, WaveRows<MAXT>, WaveBlocks<TBS, MAXT>>;
+
+  __shared__ float4 s_red[NW][DT][64];
+  __shared__ float s_m[NW][16];
+  __shared__ float s_l[NW][16];
+  __shared__ int32_t s_pref[kPersistMaxOrder + 1];
+  __shared__ int32_t s_tmp[NW];
+  __shared__ float2 s_ml[NT * 4 / D + 1];
+  __shared__ int s_last;
+  // Token rows: each wavefront's row ids (WaveRows).
+  constexpr int kRowIds = ROWS ? 64 * ((MAXT * kTile + 63) / 64) : 4;
+  __shared__ __align__(16) int32_t s_rowids[NW][kRowIds];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, col = lane & 15;
+  const int B = p.num_seqs;
+  const int span = plan_spans<NT>(p, s_pref, s_tmp, tid, gridDim.x);
+  SplitPos at = split_pos(s_pref, B, p.units, span, blockIdx.x, lane);
+  const SplitPos end = split_pos(s_pref, B, p.units, span, blockIdx.x + 1, lane);
+  const int nlb_max = (p.max_seq_len + TBS - 1) / TBS;
+  while (true) {
+    const bool last = at.seq == end.seq && at.unit == end.unit;
+    if (at.seq > end.seq || (at.seq == end.seq && at.unit > end.unit) || (last && at.off >= end.off)) break;
+    const int seq = __builtin_amdgcn_readfirstlane(at.seq), unit = __builtin_amdgcn_readfirstlane(at.unit);
+    const int a = __builtin_amdgcn_readfirstlane(at.off), upto = __builtin_amdgcn_readfirstlane(last ? end.off : -1);
+    at.off = 0;
+    if (++at.unit == p.units) {
+      at.unit = 0;
+      ++at.seq;
+    }
+    int kvh, h0, nh;
+    unit_heads(p, unit, kvh, h0, nh);
+    const uint32_t ctx = (uint32_t)p.context_lens[seq];
+    const int n = seq_tiles(p, ctx);
+    const int b = upto < 0 ? n : upto;  // the piece: tiles [a, b)
+    const int32_t* row = p.block_tables + (int64_t)seq * p.max_blocks_per_seq;
+    Blocks blk;
+    if constexpr (ROWS) blk.ids = s_rowids[wave];
+    // Block ids of the wavefront's tiles from tile t on.  The bound comes
+    // from max_seq_len rather than the context, so the first pass's loads do
+    // not wait for it; entries past the context are never used.
+    auto load_blocks = [&](int t) {
+      if constexpr (ROWS)
+        blk.load(row, __builtin_ctz((unsigned)p.block_size), p.num_blocks, p.max_seq_len, t + wave, NW, lane);
+      else
+        blk.load(row, p.num_blocks, nlb_max, 0, t * kTile, wave, NW, lane);
+    };
+    load_blocks(a);
+    uint4 qa[KSTEPS];
+    uint4 qb[SPLIT_Q ? KSTEPS : 1];
+    load_query<QT, typename MmaOf<QT, CT>::type, D, WideFp8<CT, D>::value>(p, seq, h0, nh, g, col, qa, qb);
+    const float slope = (p.alibi != nullptr && col < nh) ? p.alibi[h0 + col] * kLog2e : 0.f;
+
+    WaveAcc<D> acc;
+    acc.init();
+    using CS = typename Elem<CT>::storage;
+    const CS* kbase = static_cast<const CS*>(p.k_cache) + (int64_t)kvh * p.k_head_stride;
+    const CS* vbase = static_cast<const CS*>(p.v_cache) + (int64_t)kvh * p.v_head_stride;
+    if constexpr (ROWS) {
+      // Every head's rows end within k_rows_bytes (v_rows_bytes) of its base.
+      blk.kr = __builtin_amdgcn_make_buffer_rsrc((void*)kbase, (short)0, (int)p.k_rows_bytes, kBufferRsrcWord3);
+      blk.vr = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, (short)0, (int)p.v_rows_bytes, kBufferRsrcWord3);
+    }
+    for (int t = a; t < b;) {
+      const int te = min(b, t + MAXT * NW);
+      stream_tiles<QT, CT, D, TBS, NW, MAXT, kPartBuffers, ROWS, Blocks>(
+          p, kbase, vbase, blk, t * kTile, min(te * kTile, (int)ctx), ctx, wave, g, col, qa, qb, slope, acc);
+      t = te;
+      if (t < b) load_blocks(t);
+    }
+
+    // A piece of its item: pieces start at the workgroups whose spans begin
+    // inside it, the first of them w.
+    const bool piece = a > 0 || b < n;
+    int w = 0, pieces = 1;
+    float *so = nullptr, *sml = nullptr;
+    if (piece) {
+      const int base = p.units * s_pref[seq] + unit * (n + kItemTiles) + kItemTiles;  // of the item's tile 0
+      w = (base + kMinPiece + span - 1) / span;
+      pieces = (base + n - kMinPiece) / span - w + 2;
+      const int64_t slot = (int64_t)(2 * (int)blockIdx.x + (a == 0 ? 1 : 0)) * min(16, p.group);
+      so = p.split_o + slot * D;
+      sml = p.split_ml + slot * 2;
+    }
+    merge_store_waves<QT, D, NW, ROWS, true>(p, acc, s_red, s_m, s_l, wave, lane, g, col,
+                                             (int64_t)seq * p.num_heads + h0 + col, col < nh, so, sml);
+    if (piece) {
+      // Arrival: every wavefront's stores have completed before the count.
+      wait_stores();
+      __syncthreads();
+      if (tid == 0) s_last = arrive_last(p.split_counters + w, pieces);
+      __syncthreads();
+      if (s_last)
+        merge_pieces<QT, D, NT>(p, (int64_t)seq * p.num_heads + h0, nh, pieces, w, &s_red[0][0][0], s_ml, tid);
+    }
+    __syncthreads();  // s_red is free again
   }
 }
 
@@ -2608,6 +2921,48 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
   return hipGetLastError();
 }
 
+// The split kernel (BS = 0: token rows) where a batch has too few items to
+// balance whole ones: fewer than two per CU, each of them long enough that
+// the pieces' start-up and merge (about 10 us a launch) cost less than the
+// uneven lengths do, unless the partition kernel's grid (`other` workgroups;
+// 0: the alternative is the persistent kernel) already holds two and more per
+// CU (27 contexts of 8008 .. 9498 x 8 heads of 64, 648 workgroups: 95.9 us,
+// split 101.6).  The host knows only the longest context, so the line is
+// drawn on the tiles a CU would take if every context had it.  Measured
+// (kernel times, partition kernel and its merge -> split): token rows, 24
+// contexts of 500 .. 8000 x 8 KV heads 131 -> 92 us, 62 of 476 .. 956 x 4
+// (58 tiles a CU) 36.7 -> 33.6; FP8, 7 of 2532 .. 4634 x 32 heads of 64 (254
+// tiles) 38.2 -> 28.1; bf16, 59 of 7655 .. 22667 x 1 (327) 90 -> 71; float32,
+// 10 of 2380 .. 42476 x 2 118 -> 80.6 and 4 of 9516 .. 11370 x 8 (89) 89 ->
+// 75.5.  Below the line: bf16, 16 of 256 .. 4096 x 8 (128) 31.7 -> 32.4, FP8,
+// 15 of 1361 .. 3411 x 16 (200) 30.6 -> 32.9.
+template <class QT, class CT, int D, int BS>
+static hipError_t launch_split(const DecodeParams& p, int64_t other, hipStream_t stream, bool* launched) {
+  *launched = false;
+  if (p.split_o == nullptr || p.num_seqs > kPersistMaxOrder) return hipSuccess;
+  constexpr int64_t kMinTiles = BS == 0 ? 48 : std::is_same<CT, F32>::value ? 80 : 240;  // per CU
+  constexpr int NT = 64 * kSplitWaves;
+  static int per_cu = -1;
+  if (per_cu < 0) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, paged_decode_split_kernel<QT, CT, D, BS>, NT, 0) !=
+            hipSuccess ||
+        n <= 0)
+      n = 1;
+    per_cu = n;
+  }
+  const int64_t cus = device_cus();
+  const int64_t items = (int64_t)p.num_seqs * p.units;
+  const int64_t tiles = items * ((p.max_seq_len + kTile - 1) / kTile);
+  const int64_t grid = std::min<int64_t>({cus * per_cu, items * kMaxPieces, kSplitWorkgroups});
+  if (grid < cus || items >= 2 * cus || other >= 2 * cus || tiles < cus * kMinTiles ||
+      tiles + items * kItemTiles + grid * kMinSpan > INT32_MAX)
+    return hipSuccess;
+  *launched = true;
+  hipLaunchKernelGGL((paged_decode_split_kernel<QT, CT, D, BS>), dim3((unsigned)grid), dim3(NT), 0, stream, p);
+  return hipGetLastError();
+}
+
 template <class QT, class CT, int D, int BS>
 static hipError_t launch_persistent(const DecodeParams& p, hipStream_t stream, bool* launched) {
   *launched = false;
@@ -2637,6 +2992,17 @@ static hipError_t launch_persistent(const DecodeParams& p, hipStream_t stream, b
   const int64_t items = (int64_t)p.num_seqs * p.units;
   const int64_t grid = (int64_t)device_cus() * per_cu;
   if (grid <= 0 || items < kPersistMinItemsPerWorkgroup * grid) return hipSuccess;
+  // Between one and two items per workgroup the whole-item schedule leaves
+  // its busiest workgroup up to (2 grid - items) / (2 grid) of the longest
+  // context above the mean; the split kernel takes over where that exceeds
+  // what a split costs (about 40 tiles): FP8, 38 contexts of 1084 .. 15628 x 8
+  // (397 tiles) 128 -> 104 us; float16, 13 of 90 .. 3000 x 32 (35 tiles) 49 ->
+  // 60 us, kept whole.
+  const int64_t longest = (p.max_seq_len + kTile - 1) / kTile;
+  if (longest * (2 * grid - items) > 2 * grid * 40) {
+    const hipError_t se = launch_split<QT, CT, D, BS>(p, 0, stream, launched);
+    if (*launched || se != hipSuccess) return se;
+  }
   *launched = true;
   hipLaunchKernelGGL((paged_decode_persist_kernel<QT, CT, D, BS>), dim3((unsigned)grid), dim3(NT), 0, stream, p);
   return hipGetLastError();
@@ -2645,9 +3011,11 @@ static hipError_t launch_persistent(const DecodeParams& p, hipStream_t stream, b
 template <class QT, class CT, int D, int BS>
 static hipError_t launch_one(const DecodeParams& p, hipStream_t stream) {
   bool launched = false;
-  const hipError_t pe = launch_persistent<QT, CT, D, BS>(p, stream, &launched);
+  hipError_t pe = launch_persistent<QT, CT, D, BS>(p, stream, &launched);
   if (launched || pe != hipSuccess) return pe;
   const int64_t nwg = (int64_t)p.max_parts * p.num_seqs * p.units;
+  pe = launch_split<QT, CT, D, BS>(p, nwg, stream, &launched);
+  if (launched || pe != hipSuccess) return pe;
   // Four wavefronts per workgroup at every grid size: eight for grids of
   // at most one workgroup per CU (one long sequence) measured no faster.
   hipLaunchKernelGGL((paged_decode_part_kernel<QT, CT, D, BS, kPartWaves>), dim3((unsigned)nwg), dim3(64 * kPartWaves),
@@ -2676,9 +3044,11 @@ static hipError_t launch_bs(const DecodeParams& p, int block_size, hipStream_t s
 template <class QT, class CT, int D>
 static hipError_t launch_rows(const DecodeParams& p, hipStream_t stream) {
   bool launched = false;
-  const hipError_t pe = launch_persistent<QT, CT, D, 0>(p, stream, &launched);
+  hipError_t pe = launch_persistent<QT, CT, D, 0>(p, stream, &launched);
   if (launched || pe != hipSuccess) return pe;
   const int64_t nwg = (int64_t)p.max_parts * p.num_seqs * p.units;
+  pe = launch_split<QT, CT, D, 0>(p, nwg, stream, &launched);
+  if (launched || pe != hipSuccess) return pe;
   hipLaunchKernelGGL((paged_decode_rows_kernel<QT, CT, D>), dim3((unsigned)nwg), dim3(64 * kPartWaves), 0, stream, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.max_parts == 1) return e;

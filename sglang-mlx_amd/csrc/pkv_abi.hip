@@ -125,6 +125,14 @@ DecodeWorkspace decode_workspace_layout(int32_t num_seqs, int32_t num_heads, int
   w.total = (size_t)kCounterBytes + w.ml_bytes + w.o_bytes;
   return w;
 }
+DecodeWorkspace split_workspace_layout(int32_t num_heads, int32_t num_kv_heads, int32_t head_size) {
+  DecodeWorkspace w;
+  const size_t rows = (size_t)2 * kSplitWorkgroups * std::min(16, num_heads / num_kv_heads);
+  w.ml_bytes = rows * 2 * sizeof(float);
+  w.o_bytes = rows * head_size * sizeof(float);
+  w.total = (size_t)kCounterBytes + w.ml_bytes + w.o_bytes;
+  return w;
+}
 CascadeWorkspace cascade_workspace_layout(int32_t num_seqs, int32_t num_heads, int32_t head_size,
                                           int32_t max_chunks, int32_t max_parts) {
   CascadeWorkspace w;
@@ -218,6 +226,13 @@ size_t pkv_paged_attention_workspace_size(int32_t num_seqs, int32_t num_heads, i
   if (resolve_partition(num_seqs, num_heads, num_kv_heads, max_seq_len, 0, partition_size, &ps, &parts) != PKV_OK)
     return 0;
   return pkv::decode_workspace_layout(num_seqs, num_heads, head_size, parts).total;
+}
+
+size_t pkv_paged_attention_full_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
+                                               int32_t head_size, int32_t max_seq_len, int32_t partition_size) {
+  const size_t least = pkv_paged_attention_workspace_size(num_seqs, num_heads, num_kv_heads, head_size, max_seq_len,
+                                                          partition_size);
+  return least == 0 ? 0 : std::max(least, pkv::split_workspace_layout(num_heads, num_kv_heads, head_size).total);
 }
 
 size_t pkv_paged_attention_cascade_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
@@ -409,6 +424,16 @@ int paged_attention_impl(void* out, const void* query, const void* key_cache, co
   p.max_parts = parts;
   p.persistent = partition_size == 0 &&
                  max_seq_len <= (rows ? pkv::persist_rows_max_seq(head_size) : pkv::kPersistMaxSeq);
+  // The split kernel needs its states' room, which a workspace of
+  // pkv_paged_attention_workspace_size() bytes may lack; such calls run the
+  // other kernels.
+  const pkv::DecodeWorkspace sw = pkv::split_workspace_layout(num_heads, num_kv_heads, head_size);
+  p.split_ml = p.split_o = nullptr;
+  p.split_counters = reinterpret_cast<int32_t*>(ws);
+  if (workspace_bytes >= sw.total) {
+    p.split_ml = reinterpret_cast<float*>(ws + pkv::kCounterBytes);
+    p.split_o = reinterpret_cast<float*>(ws + pkv::kCounterBytes + sw.ml_bytes);
+  }
   p.rows = rows;
   p.block_size = block_size;
   // The paged layout's partition kernel merges its own partitions when a row
@@ -423,7 +448,7 @@ int paged_attention_impl(void* out, const void* query, const void* key_cache, co
     const int64_t k_span = ((total_rows - 1) * kbs + head_size) * 2;
     const int64_t v_span = ((total_rows - 1) * vbs + head_size) * 2;
     if (k_span > (int64_t)UINT32_MAX || v_span > (int64_t)UINT32_MAX)
-      p.persistent = 0;  // 64-bit addressing: the partition kernel
+      p.persistent = 0, p.split_o = nullptr;  // 64-bit addressing: the partition kernel
     else {
       p.k_rows_bytes = (uint32_t)k_span;
       p.v_rows_bytes = (uint32_t)v_span;

@@ -27,6 +27,10 @@ constexpr int kPersistMaxOrder = 1024;
 // with four.
 constexpr int persist_rows_max_seq(int head_size) { return head_size > 128 ? 2048 : 4096; }
 
+// Most workgroups of the split decode kernel (a state slot pair and a counter
+// each).
+constexpr int kSplitWorkgroups = 1024;
+
 struct RacParams {
   const void* key;
   const void* value;
@@ -108,6 +112,13 @@ struct DecodeParams {
   // kernel runs after it): one per (sequence, unit), zero before a launch
   // and left zero by it.
   int32_t* counters;
+  // Piece states of the split kernel (split_o null: the workspace has no room
+  // for them and the kernel is not used): per workgroup two
+  // slots of min(16, group) rows, (max, sum) in split_ml and normalised
+  // outputs in split_o, and one arrival counter, zero between launches.
+  float* split_ml;
+  float* split_o;
+  int32_t* split_counters;
 };
 
 // The partition kernel merges its own partitions (the workgroup whose state
@@ -178,6 +189,9 @@ struct DecodeWorkspace {
 };
 DecodeWorkspace decode_workspace_layout(int32_t num_seqs, int32_t num_heads, int32_t head_size,
                                         int32_t max_parts);
+// The split kernel's states take the same bytes (a call runs one or the
+// other): (max, sum) pairs, then outputs, after the counters.
+DecodeWorkspace split_workspace_layout(int32_t num_heads, int32_t num_kv_heads, int32_t head_size);
 
 // Whole-block copies (copy_blocks.hip): plane i copies block src of src[i]
 // to block dst of dst[i] for every pair of the device int64 mapping.

@@ -260,8 +260,8 @@ def _paged_attention(op, query, key_cache, value_cache, block_tables, context_le
         return out
     with torch.cuda.device(dev):
         stream = _stream(dev)
-        need = lib.pkv_paged_attention_workspace_size(B, Hq, num_kv_heads, D, max_seq_len,
-                                                      partition_size)
+        need = lib.pkv_paged_attention_full_workspace_size(B, Hq, num_kv_heads, D, max_seq_len,
+                                                           partition_size)
         if need == 0:
             _lib.check(_lib.PKV_ERR_INVALID)
         ws = _decode_scratch(dev, stream, need)

@@ -65,6 +65,7 @@ SIGNATURES = {
         _c_void_p,                                                 # stream
     ]),
     "pkv_paged_attention_workspace_size": (_size, [_i32, _i32, _i32, _i32, _i32, _i32]),
+    "pkv_paged_attention_full_workspace_size": (_size, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "pkv_paged_attention": (ctypes.c_int, [
         _c_void_p, _c_void_p, _c_void_p, _c_void_p,              # out, q, kc, vc
         _c_void_p, _c_void_p, _c_void_p,                          # block_tables, ctx, alibi
