@@ -23,11 +23,17 @@ from __future__ import annotations
 
 import ctypes
 import math
+import os
 import threading
 
 import torch
 
 from . import _lib
+
+if os.path.exists(_lib.NATIVE_PATH):
+    from . import _native
+else:  # not built: every call raises in _lib.lib()
+    _native = None
 
 _DTYPE_CODE = {torch.float32: _lib.PKV_F32, torch.float16: _lib.PKV_F16, torch.bfloat16: _lib.PKV_BF16}
 _ELEM_BYTES = {torch.float32: 4, torch.float16: 2, torch.bfloat16: 2, torch.uint8: 1}
@@ -77,6 +83,18 @@ def _as_i32(t: torch.Tensor) -> torch.Tensor:
     if t.dtype != torch.int32:
         t = t.to(torch.int32)
     return t.contiguous()
+
+
+def _done(result) -> bool:
+    """Whether the native path took a call: None and refused calls (which
+    launched nothing) go to the Python path, a HIP error is raised."""
+    if result is None:
+        return False
+    if type(result) is int:
+        if result == _lib.PKV_ERR_HIP:
+            _lib.check(result)
+        return False
+    return True
 
 
 # ---------------------------------------------------------------------------
@@ -216,6 +234,12 @@ def _plan_struct(plan, B: int, dev: torch.device):
 def _paged_attention(op, query, key_cache, value_cache, block_tables, context_lens, num_kv_heads,
                      scale, block_size, max_seq_len, alibi_slopes, partition_size, k_scale=1.0, v_scale=1.0,
                      plan=None):
+    if plan is None and _native is not None:
+        out = _native.paged_attention(_ws_cache, query, key_cache, value_cache, block_tables, context_lens,
+                                      num_kv_heads, scale, block_size, max_seq_len, alibi_slopes, partition_size,
+                                      k_scale, v_scale)
+        if _done(out):
+            return out
     for t in (query, key_cache, value_cache, block_tables, context_lens):
         _tensor(t)
     _tensor(alibi_slopes, allow_none=True)
@@ -396,6 +420,10 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, k_scale:
     caches (MHATokenPool buffers) use the token-major kernel.  uint8 caches
     hold FP8 E4M3 codes of key / k_scale and value / v_scale (x = 16).
     """
+    if _native is not None:
+        out = _native.reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, k_scale, v_scale)
+        if _done(out):
+            return out
     return _reshape_and_cache("ReshapeAndCache", key, value, key_cache, value_cache, slot_mapping, False,
                               k_scale, v_scale)
 

@@ -1,6 +1,7 @@
 """ctypes loader for libpagedkv_gfx950.so (C ABI declared in include/pagedkv.h).
 
-The shared library is the only compute path of this package.  If it has not
+The shared library is the only compute path of this package; _native.so calls
+the same library.  If it has not
 been built, ``lib()`` raises ImportError -- there is no fallback.
 """
 
@@ -12,6 +13,8 @@ import threading
 
 LIB_NAME = "libpagedkv_gfx950.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
+# The native call path of _ext.py (csrc/native_ext.cpp), built with the library.
+NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_native.so")
 
 # Status codes and enums (include/pagedkv.h).
 PKV_OK = 0
@@ -124,10 +127,11 @@ def lib() -> ctypes.CDLL:
         return _lib
     with _lock:
         if _lib is None:
-            if not os.path.exists(LIB_PATH):
-                raise ImportError(
-                    f"{LIB_PATH} is not built; run `make -C sglang-mlx_amd/csrc -j8` "
-                    "(or __graft_entry__.build())")
+            for path in (LIB_PATH, NATIVE_PATH):
+                if not os.path.exists(path):
+                    raise ImportError(
+                        f"{path} is not built; run `make -C sglang-mlx_amd/csrc -j8` "
+                        "(or __graft_entry__.build())")
             handle = ctypes.CDLL(LIB_PATH)
             for name, (res, args) in SIGNATURES.items():
                 fn = getattr(handle, name)
