@@ -5,5 +5,5 @@
 #include "paged_decode_impl.h"
 
 namespace pkv {
-template hipError_t launch_decode_typed<BF16, FP8>(const DecodeParams&, int, int, hipStream_t, bool*);
+template hipError_t launch_decode_typed<BF16, FP8>(const DecodeArgs&, int, int, hipStream_t, bool*);
 }  // namespace pkv

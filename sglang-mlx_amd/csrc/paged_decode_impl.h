@@ -2142,7 +2142,7 @@ __device__ __forceinline__ SplitPos split_pos(const int32_t* s_pref, int B, int 
 // the i-th in slot 2 (w - 1 + i), w being the workgroup whose span starts
 // with the second piece.
 template <class QT, int D, int NT>
-__device__ __forceinline__ void merge_pieces(const DecodeParams& p, int64_t row0, int nh, int pieces, int w,
+__device__ __forceinline__ void merge_pieces(const DecodeArgs& p, int64_t row0, int nh, int pieces, int w,
                                              float4* s_buf, float2* s_ml, int tid) {
   using QS = typename Elem<QT>::storage;
   constexpr int CH = D / 4, U = 4;
@@ -2221,7 +2221,7 @@ __device__ __forceinline__ void merge_pieces(const DecodeParams& p, int64_t row0
 // BS = 0: token-row caches (any block size, p.block_size), with each
 // wavefront's row ids in LDS (WaveRows); otherwise the paged layout.
 template <class QT, class CT, int D, int BS>
-__global__ __launch_bounds__(64 * kSplitWaves) void paged_decode_split_kernel(DecodeParams p) {
+__global__ __launch_bounds__(64 * kSplitWaves) void paged_decode_split_kernel(DecodeArgs p) {
   constexpr int NW = kSplitWaves;
   constexpr int NT = 64 * NW;
   constexpr int KSTEPS = Tile<D>::KSTEPS;
@@ -2922,25 +2922,34 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
 }
 
 // The split kernel (BS = 0: token rows) where a batch has too few items to
-// balance whole ones: fewer than two per CU, each of them long enough that
-// the pieces' start-up and merge (about 10 us a launch) cost less than the
-// uneven lengths do, unless the partition kernel's grid (`other` workgroups;
-// 0: the alternative is the persistent kernel) already holds two and more per
-// CU (27 contexts of 8008 .. 9498 x 8 heads of 64, 648 workgroups: 95.9 us,
-// split 101.6).  The host knows only the longest context, so the line is
-// drawn on the tiles a CU would take if every context had it.  Measured
-// (kernel times, partition kernel and its merge -> split): token rows, 24
-// contexts of 500 .. 8000 x 8 KV heads 131 -> 92 us, 62 of 476 .. 956 x 4
-// (58 tiles a CU) 36.7 -> 33.6; FP8, 7 of 2532 .. 4634 x 32 heads of 64 (254
-// tiles) 38.2 -> 28.1; bf16, 59 of 7655 .. 22667 x 1 (327) 90 -> 71; float32,
-// 10 of 2380 .. 42476 x 2 118 -> 80.6 and 4 of 9516 .. 11370 x 8 (89) 89 ->
-// 75.5.  Below the line: bf16, 16 of 256 .. 4096 x 8 (128) 31.7 -> 32.4, FP8,
-// 15 of 1361 .. 3411 x 16 (200) 30.6 -> 32.9.
+// balance whole ones or whole partitions: fewer than two items per CU, and
+// each of them long enough that the pieces' start-up and merge (about 10 us a
+// launch) cost less than the uneven grid does.  The host knows only the longest
+// context, so the line is drawn on the bytes (token rows: tiles) a CU would
+// take if every context had it.  `other`: the partition kernel's workgroups (0:
+// the alternative is the persistent kernel).  At one per CU or near two and
+// more its grid is even enough by itself; token rows take any grid below two,
+// as their partition path has a merge launch of its own.  Measured (kernel
+// times, partition kernel and its merge -> split):
+//   other   contexts x KV heads                               before   split
+//   280     140 of 3086 .. 3672 x 2, f16, D 128                101.6    86.9
+//   336     3 of 20778 .. 27908 x 16, bf16, D 96               108.3    89.4
+//   400     10 of 2380 .. 42476 x 2, f32, D 128                117.9    80.1
+//   408     17 of 2790 .. 11370 x 8, FP8, D 256                127.8    94.9
+//   384     24 of 500 .. 8000 x 8, f16 token rows, D 128       131.7    92.9
+//   416     26 of 789 .. 1869 x 8, bf16 token rows, D 80        41.7    33.4
+// and on the other side of the line:
+//   256     2 of 4617 .. 8881 x 32, f32, D 128                  86.8    90.9
+//   256     16 of 256 .. 4096 x 8, bf16, D 128 (1.0 MB a CU)    31.7    32.4
+//   384     4 of 4745 .. 9063 x 32, bf16, D 64 (1.1 MB)         44.6    50.0
+//   448     14 of 4068 .. 4646 x 16, f32, D 64                  81.1    87.0
+//   648     27 of 8008 .. 9498 x 8, bf16, D 64                  95.9   101.6
 template <class QT, class CT, int D, int BS>
-static hipError_t launch_split(const DecodeParams& p, int64_t other, hipStream_t stream, bool* launched) {
+static hipError_t launch_split(const DecodeArgs& p, int64_t other, hipStream_t stream, bool* launched) {
   *launched = false;
   if (p.split_o == nullptr || p.num_seqs > kPersistMaxOrder) return hipSuccess;
-  constexpr int64_t kMinTiles = BS == 0 ? 48 : std::is_same<CT, F32>::value ? 80 : 240;  // per CU
+  constexpr int64_t kTileBytes = (int64_t)kTile * D * 2 * Elem<CT>::kBytes;
+  constexpr int64_t kMinTiles = BS == 0 ? 48 : (std::is_same<CT, F32>::value ? 1300000 : 1900000) / kTileBytes;  // per CU
   constexpr int NT = 64 * kSplitWaves;
   static int per_cu = -1;
   if (per_cu < 0) {
@@ -2955,7 +2964,11 @@ static hipError_t launch_split(const DecodeParams& p, int64_t other, hipStream_t
   const int64_t items = (int64_t)p.num_seqs * p.units;
   const int64_t tiles = items * ((p.max_seq_len + kTile - 1) / kTile);
   const int64_t grid = std::min<int64_t>({cus * per_cu, items * kMaxPieces, kSplitWorkgroups});
-  if (grid < cus || items >= 2 * cus || other >= 2 * cus || tiles < cus * kMinTiles ||
+  // (8-token blocks above head size 128: 3 of 6866 .. 11142 x 16, float16,
+  // D 256, 81.6 us, split 84.4.)
+  if (BS == 8 && D > 128) return hipSuccess;
+  const bool uneven = other == 0 || (BS == 0 ? other < 2 * cus : other > cus && 10 * other <= 17 * cus);
+  if (!uneven || grid < cus || items >= 2 * cus || tiles < cus * kMinTiles ||
       tiles + items * kItemTiles + grid * kMinSpan > INT32_MAX)
     return hipSuccess;
   *launched = true;
@@ -2964,7 +2977,7 @@ static hipError_t launch_split(const DecodeParams& p, int64_t other, hipStream_t
 }
 
 template <class QT, class CT, int D, int BS>
-static hipError_t launch_persistent(const DecodeParams& p, hipStream_t stream, bool* launched) {
+static hipError_t launch_persistent(const DecodeArgs& p, hipStream_t stream, bool* launched) {
   *launched = false;
   if (!p.persistent) return hipSuccess;
   // The grouped kernel's two job buffers leave no register room (it would
@@ -2995,11 +3008,11 @@ static hipError_t launch_persistent(const DecodeParams& p, hipStream_t stream, b
   // Between one and two items per workgroup the whole-item schedule leaves
   // its busiest workgroup up to (2 grid - items) / (2 grid) of the longest
   // context above the mean; the split kernel takes over where that exceeds
-  // what a split costs (about 40 tiles): FP8, 38 contexts of 1084 .. 15628 x 8
-  // (397 tiles) 128 -> 104 us; float16, 13 of 90 .. 3000 x 32 (35 tiles) 49 ->
-  // 60 us, kept whole.
+  // 240 tiles: FP8, 38 contexts of 1084 .. 15628 x 8 (397 tiles) 128 -> 100 us.
+  // Below it whole items are faster: float16, 72 of 1824 .. 4900 x 4 (134) 92.9
+  // against 97.6 us; token rows, 39 of 2063 .. 3777 x 8 (92) 97.4 against 111.7.
   const int64_t longest = (p.max_seq_len + kTile - 1) / kTile;
-  if (longest * (2 * grid - items) > 2 * grid * 40) {
+  if (longest * (2 * grid - items) > 2 * grid * 240) {
     const hipError_t se = launch_split<QT, CT, D, BS>(p, 0, stream, launched);
     if (*launched || se != hipSuccess) return se;
   }
@@ -3009,7 +3022,7 @@ static hipError_t launch_persistent(const DecodeParams& p, hipStream_t stream, b
 }
 
 template <class QT, class CT, int D, int BS>
-static hipError_t launch_one(const DecodeParams& p, hipStream_t stream) {
+static hipError_t launch_one(const DecodeArgs& p, hipStream_t stream) {
   bool launched = false;
   hipError_t pe = launch_persistent<QT, CT, D, BS>(p, stream, &launched);
   if (launched || pe != hipSuccess) return pe;
@@ -3028,7 +3041,7 @@ static hipError_t launch_one(const DecodeParams& p, hipStream_t stream) {
 }
 
 template <class QT, class CT, int D>
-static hipError_t launch_bs(const DecodeParams& p, int block_size, hipStream_t stream, bool* ok) {
+static hipError_t launch_bs(const DecodeArgs& p, int block_size, hipStream_t stream, bool* ok) {
   switch (block_size) {
     case 8: return launch_one<QT, CT, D, 8>(p, stream);
     case 16: return launch_one<QT, CT, D, 16>(p, stream);
@@ -3042,7 +3055,7 @@ static hipError_t launch_bs(const DecodeParams& p, int block_size, hipStream_t s
 // token-row kernel plus the merge kernel when a sequence spans several
 // partitions.
 template <class QT, class CT, int D>
-static hipError_t launch_rows(const DecodeParams& p, hipStream_t stream) {
+static hipError_t launch_rows(const DecodeArgs& p, hipStream_t stream) {
   bool launched = false;
   hipError_t pe = launch_persistent<QT, CT, D, 0>(p, stream, &launched);
   if (launched || pe != hipSuccess) return pe;
@@ -3060,7 +3073,7 @@ static hipError_t launch_rows(const DecodeParams& p, hipStream_t stream) {
 // FP8 caches: paged 5-D layout only, head sizes that are multiples of x = 16.
 // Float32 caches: paged 5-D layout only.
 template <class QT, class CT, int D>
-static hipError_t launch_layout(const DecodeParams& p, int block_size, hipStream_t stream, bool* ok) {
+static hipError_t launch_layout(const DecodeArgs& p, int block_size, hipStream_t stream, bool* ok) {
   if constexpr (std::is_same<CT, FP8>::value) {
     if constexpr (D % 16 != 0) {
       *ok = false;
@@ -3085,7 +3098,7 @@ static hipError_t launch_layout(const DecodeParams& p, int block_size, hipStream
 }
 
 template <class QT, class CT>
-hipError_t launch_decode_typed(const DecodeParams& p, int head_size, int block_size, hipStream_t stream,
+hipError_t launch_decode_typed(const DecodeArgs& p, int head_size, int block_size, hipStream_t stream,
                                bool* ok) {
   switch (head_size) {
     case 32: return launch_layout<QT, CT, 32>(p, block_size, stream, ok);

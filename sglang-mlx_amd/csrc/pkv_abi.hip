@@ -391,7 +391,7 @@ int paged_attention_impl(void* out, const void* query, const void* key_cache, co
     return fail(PKV_ERR_INVALID, "workspace is smaller than pkv_paged_attention_workspace_size()");
   if (!aligned16(workspace)) return fail(PKV_ERR_INVALID, "workspace must be 16-byte aligned");
 
-  pkv::DecodeParams p;
+  pkv::DecodeArgs p;
   char* ws = static_cast<char*>(workspace);
   p.out = out;
   p.q = query;

@@ -1,8 +1,8 @@
 """ctypes loader for libpagedkv_gfx950.so (C ABI declared in include/pagedkv.h).
 
-The shared library is the only compute path of this package; _native.so calls
-the same library.  If it has not
-been built, ``lib()`` raises ImportError -- there is no fallback.
+The shared library is the only compute path of this package (_native.so calls
+it too).  If either has not been built, ``lib()`` raises ImportError -- there is
+no fallback.
 """
 
 from __future__ import annotations

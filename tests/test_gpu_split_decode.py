@@ -45,17 +45,17 @@ CONTEXTS = [1, 0, 15, 16, 17, 127, 128, 129, 2047, 2048, 2049, 4095, 4096, 4111,
 
 
 @pytest.mark.parametrize("rows", [False, True])
-@pytest.mark.parametrize("q,cache,Hq,Hkv,D,bs,reps", [("bfloat16", "bfloat16", 32, 8, 128, 16, 1),
-                                                      ("bfloat16", "bfloat16", 8, 8, 32, 16, 3),
-                                                      ("float16", "float16", 28, 4, 64, 32, 1),
-                                                      ("float32", "float16", 16, 16, 96, 8, 1),
-                                                      ("bfloat16", "bfloat16", 80, 4, 120, 16, 1),  # group of 20
-                                                      ("float32", "float32", 14, 2, 128, 16, 1),
-                                                      ("float32", "bfloat16", 4, 4, 256, 32, 1)])
-def test_uneven_contexts(rows, q, cache, Hq, Hkv, D, bs, reps):
+@pytest.mark.parametrize("q,cache,Hq,Hkv,D,bs", [("bfloat16", "bfloat16", 24, 6, 128, 16),
+                                                 ("float16", "float16", 42, 6, 80, 32),
+                                                 ("float32", "float16", 6, 6, 96, 8),
+                                                 ("bfloat16", "bfloat16", 60, 3, 120, 16),  # group of 20
+                                                 ("float32", "float32", 12, 6, 64, 16),
+                                                 ("float32", "bfloat16", 6, 6, 256, 32)])
+def test_uneven_contexts(rows, q, cache, Hq, Hkv, D, bs):
+    # 96 (sequence, unit) items, 384 partition workgroups.
     if rows and cache == "float32":
         pytest.skip("float32 caches are read in the paged layout")
-    ctx = CONTEXTS * reps
+    ctx = CONTEXTS
     # The last context of the list is longer than max_seq_len: a zero row.
     c = make_decode_case(7, B=len(ctx), Hq=Hq, Hkv=Hkv, D=D, block_size=bs, ctx_lo=1, ctx_hi=1, q_dtype=q,
                          cache_dtype=cache, alibi=D == 96, context_lens=ctx)
@@ -89,3 +89,12 @@ def test_blocks_outside_the_cache_are_masked():
             p = np.exp(s - s.max(axis=1, keepdims=True))
             ref = p @ vv[:, h] / (p.sum(axis=1, keepdims=True) + 1e-6)
             np.testing.assert_allclose(got[i, 4 * h:4 * h + 4], ref, atol=atol, rtol=rtol)
+
+
+def test_more_items_than_workgroups():
+    # 304 items, which the persistent kernel would take whole, a few of them
+    # long enough to be split.
+    ctx = [10000, 300, 0, 5000] + list(range(1, 290, 8))[:34]
+    c = make_decode_case(11, B=38, Hq=32, Hkv=8, D=128, block_size=16, ctx_lo=1, ctx_hi=1, context_lens=ctx)
+    atol, rtol = tolerance("bfloat16", "bfloat16")
+    np.testing.assert_allclose(run(c, False), decode_oracle(c), atol=atol, rtol=rtol)
