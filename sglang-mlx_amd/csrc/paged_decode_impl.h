@@ -2936,6 +2936,7 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
 //   336     3 of 20778 .. 27908 x 16, bf16, D 96               108.3    89.4
 //   400     10 of 2380 .. 42476 x 2, f32, D 128                117.9    80.1
 //   408     17 of 2790 .. 11370 x 8, FP8, D 256                127.8    94.9
+//   480     15 of 205 .. 3707 x 8, f32, D 256                  500.5   127.9
 //   384     24 of 500 .. 8000 x 8, f16 token rows, D 128       131.7    92.9
 //   416     26 of 789 .. 1869 x 8, bf16 token rows, D 80        41.7    33.4
 // and on the other side of the line:
@@ -2967,7 +2968,7 @@ static hipError_t launch_split(const DecodeArgs& p, int64_t other, hipStream_t s
   // (8-token blocks above head size 128: 3 of 6866 .. 11142 x 16, float16,
   // D 256, 81.6 us, split 84.4.)
   if (BS == 8 && D > 128) return hipSuccess;
-  const bool uneven = other == 0 || (BS == 0 ? other < 2 * cus : other > cus && 10 * other <= 17 * cus);
+  const bool uneven = other == 0 || (BS == 0 ? other < 2 * cus : other > cus && 10 * other <= (D > 128 ? 20 : 17) * cus);
   if (!uneven || grid < cus || items >= 2 * cus || tiles < cus * kMinTiles ||
       tiles + items * kItemTiles + grid * kMinSpan > INT32_MAX)
     return hipSuccess;
