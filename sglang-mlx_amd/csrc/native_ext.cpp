@@ -10,12 +10,17 @@
 // range.  The caller then runs the Python path, which has the general forms and
 // every error message.  A status other than success comes back as an int; for
 // a refused call (nothing was launched) the Python path runs as well.
+//
+// Other Python threads run while the output is allocated and the kernel is
+// launched, as under ctypes: a launch can wait for room in a full queue, and a
+// host callback ahead of it in the stream may need the interpreter.
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -95,8 +100,9 @@ PyObject* reshape_and_cache(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!plain(a[i])) Py_RETURN_NONE;
   double k_scale, v_scale;
   if (!as_double(a[5], k_scale) || !as_double(a[6], v_scale) || transformed()) Py_RETURN_NONE;
-  const Tensor &key = THPVariable_Unpack(a[0]), &value = THPVariable_Unpack(a[1]), &kc = THPVariable_Unpack(a[2]),
-               &vc = THPVariable_Unpack(a[3]), &slots = THPVariable_Unpack(a[4]);
+  // (Copies: the tensors stay alive while other threads run.)
+  const Tensor key = THPVariable_Unpack(a[0]), value = THPVariable_Unpack(a[1]), kc = THPVariable_Unpack(a[2]),
+               vc = THPVariable_Unpack(a[3]), slots = THPVariable_Unpack(a[4]);
   const c10::Device dev = key.device();
   if (!dev.is_cuda() || !usable(key, dev) || !usable(value, dev) || !usable(kc, dev) || !usable(vc, dev) ||
       !usable(slots, dev))
@@ -137,10 +143,14 @@ PyObject* reshape_and_cache(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t ks, vs;
   if (!row_stride(key, ks) || !row_stride(value, vs)) Py_RETURN_NONE;
   const OnDevice on(dev);
-  const int st = pkv_reshape_and_cache(
-      key.data_ptr(), value.data_ptr(), kc.data_ptr(), vc.data_ptr(), static_cast<const int32_t*>(slots.data_ptr()), N,
-      (int32_t)H, (int32_t)D, ks, vs, layout, (int32_t)bs, (int32_t)x, num_slots, kv, cc, (float)k_scale,
-      (float)v_scale, c10::hip::getCurrentHIPStream(dev.index()).stream());
+  int st;
+  {
+    pybind11::gil_scoped_release release;
+    st = pkv_reshape_and_cache(
+        key.data_ptr(), value.data_ptr(), kc.data_ptr(), vc.data_ptr(), static_cast<const int32_t*>(slots.data_ptr()),
+        N, (int32_t)H, (int32_t)D, ks, vs, layout, (int32_t)bs, (int32_t)x, num_slots, kv, cc, (float)k_scale,
+        (float)v_scale, c10::hip::getCurrentHIPStream(dev.index()).stream());
+  }
   if (st != PKV_OK) return PyLong_FromLong(st);
   PyObject* out = PyList_New(2);
   if (out == nullptr) return nullptr;
@@ -165,20 +175,21 @@ PyObject* paged_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!as_int(a[6], Hkv) || !as_double(a[7], scale) || !as_int(a[8], bs) || !as_int(a[9], max_seq) ||
       !as_int(a[11], partition) || !as_double(a[12], k_scale) || !as_double(a[13], v_scale) || transformed())
     Py_RETURN_NONE;
-  const Tensor &q = THPVariable_Unpack(a[1]), &kc = THPVariable_Unpack(a[2]), &vc = THPVariable_Unpack(a[3]),
-               &bt = THPVariable_Unpack(a[4]), &lens = THPVariable_Unpack(a[5]);
+  const Tensor q = THPVariable_Unpack(a[1]), kc = THPVariable_Unpack(a[2]), vc = THPVariable_Unpack(a[3]),
+               bt = THPVariable_Unpack(a[4]), lens = THPVariable_Unpack(a[5]);
   const c10::Device dev = q.device();
   if (!dev.is_cuda() || !usable(q, dev) || !usable(kc, dev) || !usable(vc, dev) || !usable(bt, dev) ||
       !usable(lens, dev))
     Py_RETURN_NONE;
+  Tensor slopes;
   const float* alibi = nullptr;
   if (a[10] != Py_None) {
     if (!plain(a[10])) Py_RETURN_NONE;
-    const Tensor& t = THPVariable_Unpack(a[10]);
-    if (!usable(t, dev) || t.scalar_type() != at::kFloat || t.dim() != 1 || !t.is_contiguous() || q.dim() != 3 ||
-        t.size(0) != q.size(1))
+    slopes = THPVariable_Unpack(a[10]);
+    if (!usable(slopes, dev) || slopes.scalar_type() != at::kFloat || slopes.dim() != 1 || !slopes.is_contiguous() ||
+        q.dim() != 3 || slopes.size(0) != q.size(1))
       Py_RETURN_NONE;
-    alibi = static_cast<const float*>(t.data_ptr());
+    alibi = static_cast<const float*>(slopes.data_ptr());
   }
   if (q.dim() != 3 || !i32_contiguous(bt, 2) || !i32_contiguous(lens, 1)) Py_RETURN_NONE;
   const int64_t B = q.size(0), Hq = q.size(1), D = q.size(2);
@@ -228,13 +239,18 @@ PyObject* paged_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor ws = THPVariable_Unpack(held);
   if (ws.scalar_type() != at::kByte || (size_t)ws.numel() < need) Py_RETURN_NONE;
   const OnDevice on(dev);
-  Tensor out = at::empty({B, Hq, D}, q.options());
-  const int st = pkv_paged_attention(
-      out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), static_cast<const int32_t*>(bt.data_ptr()),
-      static_cast<const int32_t*>(lens.data_ptr()), alibi, (int32_t)B, (int32_t)Hq, (int32_t)Hkv, (int32_t)D,
-      (int32_t)bs, (int32_t)bt.size(1), (int32_t)max_seq, kc.size(0), (float)scale, q.stride(0), kc.stride(0), khs,
-      vc.stride(0), vhs, layout, (int32_t)partition, ws.data_ptr(), (size_t)ws.numel(), qc, cc, (float)k_scale,
-      (float)v_scale, stream);
+  Tensor out;
+  int st;
+  {
+    pybind11::gil_scoped_release release;
+    out = at::empty({B, Hq, D}, q.options());
+    st = pkv_paged_attention(
+        out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), static_cast<const int32_t*>(bt.data_ptr()),
+        static_cast<const int32_t*>(lens.data_ptr()), alibi, (int32_t)B, (int32_t)Hq, (int32_t)Hkv, (int32_t)D,
+        (int32_t)bs, (int32_t)bt.size(1), (int32_t)max_seq, kc.size(0), (float)scale, q.stride(0), kc.stride(0), khs,
+        vc.stride(0), vhs, layout, (int32_t)partition, ws.data_ptr(), (size_t)ws.numel(), qc, cc, (float)k_scale,
+        (float)v_scale, stream);
+  }
   if (st != PKV_OK) return PyLong_FromLong(st);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS

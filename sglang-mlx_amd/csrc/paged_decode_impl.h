@@ -44,6 +44,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 
 #include "pkv_fp8.h"
 #include "pkv_launch.h"
@@ -2879,16 +2880,26 @@ __global__ __launch_bounds__(64 * kMergeWaves) void paged_decode_reduce_kernel(D
 // ---------------------------------------------------------------------------
 
 // Multiprocessor count of the current device, cached per device.
+// (Calls run in several threads at once: the cache is atomic, and the resident
+// workgroups of a kernel are static constants.)
 inline int device_cus() {
-  static int cache[64] = {0};
+  static std::atomic<int> cache[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cache[dev] == 0) {
-    int n = 0;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cache[dev] = n;
+    cache[dev].store(n, std::memory_order_relaxed);
   }
-  return cache[dev];
+  return n;
+}
+
+// Workgroups of a kernel that one CU holds at once.
+template <class Kernel>
+inline int resident_per_cu(Kernel kernel, int threads) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0) != hipSuccess || n <= 0) return 1;
+  return n;
 }
 
 // Launches the persistent kernel (BS = 0: token rows) when the batch has
@@ -2903,15 +2914,7 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
   constexpr int NW = GroupShape<CT, D>::kWaves, NB = kGroupBuffers;
   if (p.slices != 1 || p.group * S > 16 || p.max_seq_len > group_max_seq<NW>()) return hipSuccess;
   constexpr int NT = 64 * NW;
-  static int per_cu = -1;
-  if (per_cu < 0) {
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, paged_decode_group_kernel<QT, CT, D, BS, S, NW, NB>, NT, 0) !=
-            hipSuccess ||
-        n <= 0)
-      n = 1;
-    per_cu = n;
-  }
+  static const int per_cu = resident_per_cu(paged_decode_group_kernel<QT, CT, D, BS, S, NW, NB>, NT);
   const int64_t items = (int64_t)((p.num_seqs + S - 1) / S) * p.num_kv_heads;
   const int64_t grid = (int64_t)device_cus() * std::min(per_cu, GroupShape<CT, D>::kPerCu);
   if (grid <= 0 || items < 2 * (int64_t)device_cus()) return hipSuccess;
@@ -2952,15 +2955,7 @@ static hipError_t launch_split(const DecodeArgs& p, int64_t other, hipStream_t s
   constexpr int64_t kTileBytes = (int64_t)kTile * D * 2 * Elem<CT>::kBytes;
   constexpr int64_t kMinTiles = BS == 0 ? 48 : (std::is_same<CT, F32>::value ? 1300000 : 1900000) / kTileBytes;  // per CU
   constexpr int NT = 64 * kSplitWaves;
-  static int per_cu = -1;
-  if (per_cu < 0) {
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, paged_decode_split_kernel<QT, CT, D, BS>, NT, 0) !=
-            hipSuccess ||
-        n <= 0)
-      n = 1;
-    per_cu = n;
-  }
+  static const int per_cu = resident_per_cu(paged_decode_split_kernel<QT, CT, D, BS>, NT);
   const int64_t cus = device_cus();
   const int64_t items = (int64_t)p.num_seqs * p.units;
   const int64_t tiles = items * ((p.max_seq_len + kTile - 1) / kTile);
@@ -2990,15 +2985,7 @@ static hipError_t launch_persistent(const DecodeArgs& p, hipStream_t stream, boo
     if (*launched || ge != hipSuccess) return ge;
   }
   constexpr int NT = 64 * Persist<D, BS == 0>::kWaves;
-  static int per_cu = -1;  // resident workgroups per CU for this instantiation
-  if (per_cu < 0) {
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, paged_decode_persist_kernel<QT, CT, D, BS>, NT, 0) !=
-            hipSuccess ||
-        n <= 0)
-      n = 1;
-    per_cu = n;
-  }
+  static const int per_cu = resident_per_cu(paged_decode_persist_kernel<QT, CT, D, BS>, NT);
   // Whole (sequence, unit) items, from one per resident workgroup; fewer,
   // longer items go to the partition path.  The grid never exceeds what is
   // resident at once, which the snake schedule assumes for its balance (not

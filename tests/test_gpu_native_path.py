@@ -1,7 +1,11 @@
 """The native call path (_native.so) against the Python path it stands in for:
 plain calls are taken and give the same bytes, every other form is handed back
-and gives what the Python path gives, refusals keep their messages, and
-streams, tensor subclasses and function modes are as before."""
+and gives what the Python path gives, refusals keep their messages, streams,
+tensor subclasses and function modes are as before, and other threads run
+during a call."""
+
+import sys
+import threading
 
 import pytest
 import torch
@@ -152,3 +156,37 @@ def test_side_stream_uses_its_own_scratch():
     side.synchronize()
     assert all(torch.equal(o, ref) for o in outs)
     assert (0, side.cuda_stream) in _ext._ws_cache
+
+
+@pytest.mark.parametrize("call", ["decode", "append"])
+def test_other_threads_run_during_a_call(call):
+    # With this switch interval a thread that waits for the interpreter gets it
+    # only where the running thread gives it up by itself.
+    args = decode_args() if call == "decode" else append_args()
+    if call == "decode":
+        _ext.paged_attention_v1(*args)  # (allocates the scratch)
+        native, full = _ext._native.paged_attention, (_ext._ws_cache, *args, None, 0, 1.0, 1.0)
+    else:
+        native, full = _ext._native.reshape_and_cache, (*args, 1.0, 1.0)
+    torch.cuda.synchronize()
+    ran, go = [], threading.Event()
+
+    def other():
+        go.wait()
+        ran.append(True)
+
+    t = threading.Thread(target=other)
+    t.start()
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        go.set()
+        for calls in range(20000):
+            if ran:
+                break
+            assert native(*full) is not None
+    finally:
+        sys.setswitchinterval(interval)
+    seen = bool(ran)
+    t.join()
+    assert seen
