@@ -256,11 +256,28 @@ PyObject* paged_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// (stream handle) -> a number that names the HIP graph capture under way on
+// the stream, 0 if there is none.
+PyObject* capture_id(PyObject*, PyObject* handle) {
+  HANDLE_TH_ERRORS
+  const unsigned long long h = PyLong_AsUnsignedLongLong(handle);
+  if (PyErr_Occurred()) return nullptr;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(reinterpret_cast<hipStream_t>((uintptr_t)h), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();  // the legacy stream beside another stream's capture: it captures nothing itself
+    return PyLong_FromLong(0);
+  }
+  return PyLong_FromUnsignedLongLong(status == hipStreamCaptureStatusNone ? 0 : id + 1);
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
     {"reshape_and_cache", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(reshape_and_cache)),
      METH_FASTCALL, nullptr},
     {"paged_attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(paged_attention)), METH_FASTCALL,
      nullptr},
+    {"capture_id", capture_id, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", "Append and decode calls without the Python checks.", -1,

@@ -99,22 +99,46 @@ def _done(result) -> bool:
 
 # ---------------------------------------------------------------------------
 # Decode scratch, one buffer per (device, stream).  Its first
-# PKV_COUNTER_BYTES are arrival counters that start at zero (a new buffer is
-# zero-filled) and that every call leaves at zero; the rest is read only
+# PKV_COUNTER_BYTES are arrival counters that start at zero (cleared when the
+# buffer is made) and that every call leaves at zero; the rest is read only
 # where the same launch wrote it.  So calls ordered on one stream share it
 # whatever their shapes.
+#
+# HIP graphs: a call captured on a stream that has its buffer already uses that
+# buffer, so an outgrown buffer is kept for the graphs that hold its address
+# (sizes are powers of two: all of them together are smaller than the current
+# one).  Otherwise the buffer is made inside the capture, from the graph's
+# memory, and its clearing is a node of that graph that only runs when the
+# graph does: such a buffer serves the rest of the same capture and no other
+# call.
 # ---------------------------------------------------------------------------
 _ws_lock = threading.Lock()
 _ws_cache: dict = {}
+_ws_captured: dict = {}  # (device, stream) -> (capture, buffer)
+_ws_outgrown: list = []
+
+
+def _new_scratch(dev: torch.device, scratch_bytes: int) -> torch.Tensor:
+    scratch = torch.empty(1 << max(17, (scratch_bytes - 1).bit_length()), dtype=torch.uint8, device=dev)
+    scratch[:_lib.PKV_COUNTER_BYTES].zero_()
+    return scratch
 
 
 def _decode_scratch(dev: torch.device, stream: int, scratch_bytes: int) -> torch.Tensor:
     key = (dev.index, stream)
     with _ws_lock:
         scratch = _ws_cache.get(key)
-        if scratch is None or scratch.numel() < scratch_bytes:
-            scratch = torch.zeros(max(scratch_bytes, 1 << 17), dtype=torch.uint8, device=dev)
-            _ws_cache[key] = scratch
+        if scratch is not None and scratch.numel() >= scratch_bytes:
+            return scratch
+        capture = _native.capture_id(stream)
+        if capture:
+            held = _ws_captured.get(key)
+            if held is None or held[0] != capture or held[1].numel() < scratch_bytes:
+                held = _ws_captured[key] = (capture, _new_scratch(dev, scratch_bytes))
+            return held[1]
+        if scratch is not None:
+            _ws_outgrown.append(scratch)
+        scratch = _ws_cache[key] = _new_scratch(dev, scratch_bytes)
         return scratch
 
 
