@@ -30,7 +30,7 @@ import torch
 
 from . import _lib
 
-if os.path.exists(_lib.NATIVE_PATH):
+if os.path.exists(_lib.LIB_PATH) and os.path.exists(_lib.NATIVE_PATH):
     from . import _native
 else:  # not built: every call raises in _lib.lib()
     _native = None
