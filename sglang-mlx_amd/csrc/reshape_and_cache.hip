@@ -245,8 +245,15 @@ __device__ __forceinline__ typename Vec8<CT>::type load_v_task(const typename El
   }
 }
 
-template <class KT, class CT, int BS, bool SPLIT>
+// FEW: a call of fewer than BS tokens, in which no run exists: one window, no
+// search for runs, SPLIT's division of the work.  Such a call is a chain of
+// round trips (kernel arguments, slots, stores), and a search between them
+// shows: single tokens, kernel times, 2 heads x 64 1.84 us in a kernel without
+// any search, 2.20 with it and all of SPLIT's wavefronts, 1.70 in this form;
+// 8 x 128, blocks of 8, 2.44, 2.70 and 2.42.
+template <class KT, class CT, int BS, bool SPLIT, bool FEW>
 __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int hg, int head_groups) {
+  static_assert(SPLIT || !FEW, "few tokens are split over workgroups");
   using KS = typename Elem<KT>::storage;
   using CS = typename Elem<CT>::storage;
   constexpr bool F8 = std::is_same<CT, FP8>::value;
@@ -281,11 +288,14 @@ __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int 
     own_v1 = vsrc[min(lane + 64, D - 1)];
   }
 
-  int64_t prev, run;
-  int lane_slot;
-  rac_window_runs<BS>(p, window, lane, prev, run, lane_slot);
+  int64_t prev = -1, run = -1;
+  int lane_slot;  // lanes BS .. 2 BS - 1: the window's slots
+  if constexpr (FEW)
+    lane_slot = lane >= BS && lane - BS < p.num_tokens ? p.slot_mapping[lane - BS] : -1;
+  else
+    rac_window_runs<BS>(p, window, lane, prev, run, lane_slot);
 
-  if (run >= 0) {
+  if (!FEW && run >= 0) {
     const int units = D * (BS / 8);  // tasks per head
     const int64_t blk = p.slot_mapping[run] / BS;
     const KS* k0 = key + run * p.key_stride;
@@ -315,7 +325,7 @@ __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int 
   }
 
   // The window's other tokens.
-  const int64_t s0 = prev >= 0 ? prev + BS : w0;  // prev + BS > w0
+  const int64_t s0 = prev >= 0 ? prev + BS : w0;  // prev + BS >= w0
   const int64_t s1 = run >= 0 ? run : min(w0 + BS, p.num_tokens);
   if (s0 >= s1) return;
   const int lane0 = (int)(s0 - w0) + BS;  // the lane that holds token s0's slot
@@ -607,17 +617,23 @@ constexpr int64_t kWindowSplitBelow = 8192;
 template <class KT, class CT, int BS>
 static hipError_t launch_window_bs(const RacParams& p, hipStream_t stream) {
   const int64_t windows = (p.num_tokens + BS - 1) / BS;
-  if (p.num_tokens * p.num_heads < kWindowSplitBelow) {
+  if (p.num_tokens < BS && p.num_tokens * p.num_heads < kWindowSplitBelow) {
+    // Only wavefronts (FP8: threads) that have a token.
+    const int tokens = (int)p.num_tokens;
+    const int parts = std::is_same<CT, FP8>::value ? (tokens * p.head_size + 2047) / 2048 : (tokens + 3) / 4;
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, true, true>),
+                       dim3((unsigned)p.num_heads, (unsigned)parts), dim3(256), 0, stream, p, 1, p.num_heads);
+  } else if (p.num_tokens * p.num_heads < kWindowSplitBelow) {
     const int parts = std::is_same<CT, FP8>::value ? std::max(1, BS * p.head_size / 2048) : BS / 4;
-    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, true>),
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, true, false>),
                        dim3((unsigned)(windows * p.num_heads), (unsigned)parts), dim3(256), 0, stream, p, 1,
                        p.num_heads);
   } else {
     const int units = p.head_size * (BS / 8);
     const int hg = std::min(p.num_heads, (256 + units - 1) / units);
     const int groups = (p.num_heads + hg - 1) / hg;
-    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, false>), dim3((unsigned)(windows * groups)), dim3(256), 0,
-                       stream, p, hg, groups);
+    hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, false, false>), dim3((unsigned)(windows * groups)),
+                       dim3(256), 0, stream, p, hg, groups);
   }
   return hipGetLastError();
 }

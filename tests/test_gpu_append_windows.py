@@ -41,10 +41,11 @@ def window_slots(bs, nb, seed):
     return np.array(out, dtype=np.int32)
 
 
-def check(bs, H, D, kv_dtype, cache_dtype, seed, scales=(1.0, 1.0), values=None):
+def check(bs, H, D, kv_dtype, cache_dtype, seed, scales=(1.0, 1.0), values=None, nb=None, slots=None):
     x = 16 if cache_dtype == FP8 else 8
-    nb = 3 * bs + 16
-    slots = window_slots(bs, nb, seed)
+    if slots is None:
+        nb = 3 * bs + 16
+        slots = window_slots(bs, nb, seed)
     rng = np.random.default_rng(seed)
     N = len(slots)
     if values is None:
@@ -90,3 +91,19 @@ def test_fp8(bs, H, D, kv_dtype, scales):
     with np.errstate(over="ignore"):
         values = (QUOTIENTS * np.float32(scales[0])).astype(np.float32)
     check(bs, H, D, kv_dtype, FP8, seed=bs + D, scales=scales, values=values)
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("H,D", [(1, 128), (3, 80), (2, 256)])
+@pytest.mark.parametrize("pair", [("bfloat16", "bfloat16"), ("float32", "float16"), ("bfloat16", FP8)])
+def test_fewer_tokens_than_a_block(bs, H, D, pair):
+    nb = 9
+    rng = np.random.default_rng(bs + D)
+    scales = (0.05, 0.02) if pair[1] == FP8 else (1.0, 1.0)
+    for n in (1, 2, bs // 2 + 1, bs - 1):
+        whole = np.arange(3 * bs, 3 * bs + n)  # a block's first tokens in order
+        mixed = rng.permutation(nb * bs)[:n]
+        if n > 2:
+            mixed[[0, n // 2]] = -1, nb * bs + 1
+        for slots in (whole, mixed, np.arange(nb * bs - n, nb * bs)):
+            check(bs, H, D, *pair, seed=n, scales=scales, nb=nb, slots=slots.astype(np.int32))
