@@ -245,9 +245,10 @@ __device__ __forceinline__ typename Vec8<CT>::type load_v_task(const typename El
   }
 }
 
-// FEW: a call of fewer than BS tokens, in which no run exists: one window, no
-// search for runs, SPLIT's division of the work.  Such a call is a chain of
-// round trips (kernel arguments, slots, stores), and a search between them
+// FEW: every token on its own, in runs too, without the search for them, and
+// SPLIT's division of the work: calls of fewer than BS tokens, in which no run
+// exists, and small ones (the line is at window_few).  Such a call is a chain
+// of round trips (kernel arguments, slots, stores), and a search between them
 // shows: single tokens, kernel times, 2 heads x 64 1.84 us in a kernel without
 // any search, 2.20 with it and all of SPLIT's wavefronts, 1.70 in this form;
 // 8 x 128, blocks of 8, 2.44, 2.70 and 2.42.
@@ -291,13 +292,13 @@ __global__ __launch_bounds__(256) void rac_paged_window_kernel(RacParams p, int 
   int64_t prev = -1, run = -1;
   int lane_slot;  // lanes BS .. 2 BS - 1: the window's slots
   if constexpr (FEW)
-    lane_slot = lane >= BS && lane - BS < p.num_tokens ? p.slot_mapping[lane - BS] : -1;
+    lane_slot = lane >= BS && lane < 2 * BS && w0 + lane - BS < p.num_tokens ? p.slot_mapping[w0 + lane - BS] : -1;
   else
     rac_window_runs<BS>(p, window, lane, prev, run, lane_slot);
 
   if (!FEW && run >= 0) {
     const int units = D * (BS / 8);  // tasks per head
-    const int64_t blk = p.slot_mapping[run] / BS;
+    const int64_t blk = __builtin_amdgcn_readlane(lane_slot, BS + (int)(run - w0)) / BS;
     const KS* k0 = key + run * p.key_stride;
     const KS* v0 = val + run * p.value_stride;
     const int64_t region0 = (blk * p.num_heads + h0) * (int64_t)D * BS;
@@ -609,20 +610,46 @@ __global__ __launch_bounds__(256) void rac_fp8_paged5d_kernel(RacParams p) {
 // many workgroups as give every token (FP8: eight elements) a wavefront
 // (thread) of its own; the split index is the grid's slower one, so that the
 // parts of a window mostly share an XCD and its L2 combines a block's tokens
-// into lines (902 ragged tokens of 32-token blocks 11.0 -> 5.7 us).  The line:
+// into lines (902 ragged tokens of 32-token blocks: 5.7 us, as with a wavefront
+// per token and head; whole windows per workgroup 11.0).  The line:
 // the (token, head) wavefronts that the chip holds at once (32 per CU).
 // (Four heads of one token per workgroup instead of four tokens of one head:
 // 500 scattered windows of 16 5.2 -> 7.4 us.)
 constexpr int64_t kWindowSplitBelow = 8192;
+// Whether a call takes the FEW form: in fewer than BS tokens no run exists, and
+// below the line writing a run's tokens one by one costs less than finding it.
+// FP8 codes always search: a run's tasks encode half as often (64 tokens in
+// order, 8 x 128, blocks of 16: 3.06 us, FEW 3.73).  Measured with every token
+// in a run (device time of captured calls, search -> FEW), bf16:
+//   32 x 8 x 64, blocks of 32 (16K elements)    2.66  2.10
+//   96 x 8 x 128, blocks of 16 (98K)            2.54  2.26
+//   128 x 8 x 128, blocks of 32 (131K)          2.85  2.54
+//   64 x 8 x 256, blocks of 32 (131K)           2.76  2.92
+//   384 x 8 x 64, blocks of 32 (197K)           2.87  3.02
+//   256 x 8 x 128, blocks of 16 (262K)          2.66  2.80
+// and from float32, whose run tasks load twice the bytes:
+//   128 x 8 x 128, blocks of 16 (131K)          2.97  2.38
+//   256 x 8 x 128, blocks of 16 (262K)          3.11  2.81
+//   512 x 8 x 128, blocks of 16 (524K)          3.26  3.81
+// Scattered tokens take 0.2 to 0.4 us less in the FEW form at every size.
+template <class KT, class CT, int BS>
+static bool window_few(const RacParams& p) {
+  if (p.num_tokens * p.num_heads >= kWindowSplitBelow) return false;
+  if (p.num_tokens < BS) return true;
+  if (std::is_same<CT, FP8>::value) return false;
+  const int64_t line = (std::is_same<KT, F32>::value ? 1 << 18 : 1 << 17) / (p.head_size > 128 ? 2 : 1);
+  return p.num_tokens * p.num_heads * p.head_size <= line;
+}
 template <class KT, class CT, int BS>
 static hipError_t launch_window_bs(const RacParams& p, hipStream_t stream) {
   const int64_t windows = (p.num_tokens + BS - 1) / BS;
-  if (p.num_tokens < BS && p.num_tokens * p.num_heads < kWindowSplitBelow) {
-    // Only wavefronts (FP8: threads) that have a token.
-    const int tokens = (int)p.num_tokens;
+  if (window_few<KT, CT, BS>(p)) {
+    // A call of one window: only wavefronts (FP8: threads) that have a token.
+    const int tokens = (int)std::min<int64_t>(p.num_tokens, BS);
     const int parts = std::is_same<CT, FP8>::value ? (tokens * p.head_size + 2047) / 2048 : (tokens + 3) / 4;
     hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, true, true>),
-                       dim3((unsigned)p.num_heads, (unsigned)parts), dim3(256), 0, stream, p, 1, p.num_heads);
+                       dim3((unsigned)(windows * p.num_heads), (unsigned)parts), dim3(256), 0, stream, p, 1,
+                       p.num_heads);
   } else if (p.num_tokens * p.num_heads < kWindowSplitBelow) {
     const int parts = std::is_same<CT, FP8>::value ? std::max(1, BS * p.head_size / 2048) : BS / 4;
     hipLaunchKernelGGL((rac_paged_window_kernel<KT, CT, BS, true, false>),

@@ -107,3 +107,23 @@ def test_fewer_tokens_than_a_block(bs, H, D, pair):
             mixed[[0, n // 2]] = -1, nb * bs + 1
         for slots in (whole, mixed, np.arange(nb * bs - n, nb * bs)):
             check(bs, H, D, *pair, seed=n, scales=scales, nb=nb, slots=slots.astype(np.int32))
+
+
+@pytest.mark.parametrize("bs,N,H,D,kv", [
+    # Either side of the lines: one by one up to 2^17 (from float32 2^18)
+    # elements, half of that above head size 128; then the search for runs.
+    (16, 128, 8, 128, "bfloat16"), (16, 129, 8, 128, "bfloat16"), (32, 64, 8, 256, "bfloat16"),
+    (32, 32, 8, 256, "bfloat16"), (8, 33, 8, 256, "bfloat16"), (32, 1023, 1, 128, "bfloat16"),
+    (16, 256, 8, 128, "float32"), (16, 257, 8, 128, "float32"), (32, 131, 8, 256, "float32")])
+def test_small_calls_with_whole_blocks(bs, N, H, D, kv):
+    # Prompts that fill whole blocks and end inside one, and a first token at
+    # an offset.
+    rng = np.random.default_rng(N + bs)
+    nb = 2 * (N // bs) + 12
+    free = (rng.permutation(nb - 1) + 1).tolist()
+    slots = [free.pop() * bs + bs - 1]
+    while len(slots) < N:
+        n = int(rng.integers(1, 3 * bs))
+        at = [free.pop() for _ in range(min(-(-n // bs), len(free)))] if free else []
+        slots += [b * bs + t for b in at for t in range(bs)][:n] if at else [-1] * n
+    check(bs, H, D, kv, "float16" if kv == "float32" else kv, seed=N, nb=nb, slots=np.array(slots[:N], dtype=np.int32))
