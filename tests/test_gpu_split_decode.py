@@ -1,19 +1,32 @@
 """GPU parity of the split decode kernel: batches of few, long and uneven
 contexts whose items are computed in pieces that workgroups merge.  Contexts
-around the tile and pass sizes, empty and over-long contexts between live ones,
-16- and 32-bit caches and token rows, blocks outside the cache, a repeated call on the same scratch (arrival counters return to zero),
-and the same result from run to run."""
+around the tile and pass sizes, pieces longer than a pass, empty and over-long
+contexts between live ones, 16- and 32-bit and FP8 caches, token rows of one and
+of several tokens a block, explicit partition sizes, blocks outside the cache,
+a workspace without room for the pieces, a
+repeated call on the same scratch (arrival counters return to zero), and the
+same result from run to run.  Every case checks that the kernel ran."""
 
 import numpy as np
 import pytest
 import torch
 
 from oracle import pagedkv_oracle as orc
-from pkv_cases import decode_oracle, make_decode_case, tolerance
+from pkv_cases import X_OF, decode_oracle, make_decode_case, normal, tolerance
+from pkv_kernels import kernels_of
 from pkv_torch import to_f64, to_index, to_torch
-from sglang_mlx_amd import kernels
+from sglang_mlx_amd import _lib, kernels
 
 pytestmark = pytest.mark.gpu
+FP8 = "fp8_e4m3"
+KS, VS = 0.05, 0.02
+
+
+def split_grid(call):
+    """Workgroups of the split kernel that call() launches, and no other kernel."""
+    (name, grid), = kernels_of(call)
+    assert "split_kernel" in name, name
+    return grid
 
 
 def rows_of(case):
@@ -37,6 +50,7 @@ def run(c, rows):
     alibi = None if c.alibi is None else torch.from_numpy(c.alibi).cuda()
     outs = [kernels.paged_attention_v1(*args, alibi_slopes=alibi) for _ in range(3)]
     torch.cuda.synchronize()
+    split_grid(lambda: kernels.paged_attention_v1(*args, alibi_slopes=alibi))
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     return to_f64(outs[0])
 
@@ -98,3 +112,102 @@ def test_more_items_than_workgroups():
     c = make_decode_case(11, B=38, Hq=32, Hkv=8, D=128, block_size=16, ctx_lo=1, ctx_hi=1, context_lens=ctx)
     atol, rtol = tolerance("bfloat16", "bfloat16")
     np.testing.assert_allclose(run(c, False), decode_oracle(c), atol=atol, rtol=rtol)
+
+
+def pool_case(q, cache, Hq, Hkv, D, bs, ctx, max_seq_len, flash=False, seed=1, nb=96):
+    """Contexts over a small pool whose blocks many tables share: (call arguments,
+    reference).  flash: token rows [nb, bs, Hkv, D]."""
+    rng = np.random.default_rng(seed)
+    x = 16 if cache == FP8 else X_OF[cache]
+    shapes = [(nb, bs, Hkv, D)] * 2 if flash else [(nb, Hkv, D // x, bs, x), (nb, Hkv, D, bs)]
+    if cache == FP8:
+        k, v = (orc.fp8_e4m3_encode(rng.standard_normal(s, dtype=np.float32) * 20) for s in shapes)
+        scales = dict(k_scale=KS, v_scale=VS)
+    else:
+        k, v = (normal(rng, s, cache) for s in shapes)
+        scales = {}
+    ctx = np.asarray(ctx, dtype=np.int32)
+    qs = normal(rng, (len(ctx), Hq, D), q)
+    table = rng.integers(0, nb, size=(len(ctx), -(-max_seq_len // bs))).astype(np.int32)
+    scale = D ** -0.5
+    args = (to_torch(qs, q), to_torch(k, cache), to_torch(v, cache), to_index(table), to_index(ctx), Hkv, scale, bs,
+            max_seq_len)
+    if flash:  # the reference reads the paged layout
+        k = k.reshape(nb, bs, Hkv, D // x, x).transpose(0, 2, 3, 1, 4)
+        v = v.transpose(0, 2, 3, 1)
+    ref = orc.paged_attention(qs, k, v, table, ctx, Hkv, scale, bs, max_seq_len, None, q, cache, **scales)
+    return args, scales, ref
+
+
+def check(q, cache, Hq, Hkv, D, bs, ctx, max_seq_len, partition=0, **kw):
+    args, scales, ref = pool_case(q, cache, Hq, Hkv, D, bs, ctx, max_seq_len, **kw)
+
+    def call():
+        if partition:
+            return kernels.paged_attention_v2(*args, partition_size=partition, **scales)
+        return kernels.paged_attention_v1(*args, **scales)
+
+    out = call()
+    assert torch.equal(out, call())
+    atol, rtol = tolerance(q, "float16" if cache == FP8 else cache)
+    np.testing.assert_allclose(to_f64(out), ref, atol=atol, rtol=rtol)
+    return split_grid(call)
+
+
+@pytest.mark.parametrize("q", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("D,bs", [(128, 8), (128, 32), (256, 16), (256, 32)])
+def test_fp8(q, D, bs):
+    # Head size 256: in the partition kernel's place; 128: in the persistent
+    # kernel's (the line lies above what the partition kernel takes).
+    if D == 256:
+        check(q, FP8, 12, 6, D, bs, CONTEXTS, 16384)
+    else:
+        check(q, FP8, 16, 8, D, bs, [15000, 16, 1, 0, 9000, 4097, 16400] + [33] * 31, 16384)
+
+
+@pytest.mark.parametrize("q,cache", [("float16", "float16"), ("float32", "float32"), ("bfloat16", FP8)])
+@pytest.mark.parametrize("bs", [32, 16])
+def test_partition_sizes(q, cache, bs):
+    for partition in (512, 4096):
+        check(q, cache, 12, 6, 256, bs, CONTEXTS, 16384, partition=partition)
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+def test_rows_of_blocks(bs):
+    check("float16", "float16", 12, 6, 128, bs, CONTEXTS, 16384, flash=True)
+
+
+@pytest.mark.parametrize("flash", [False, True])
+def test_pieces_of_several_passes(flash):
+    # A workgroup holds the block ids of 4096 tokens (row ids of 2048) at a
+    # time; here its mean load alone is more.
+    ctx = [12288 - 7 * i for i in range(16)] if flash else [16384 - 50 * i for i in range(38)]
+    grid = check("bfloat16", "bfloat16", 8, 8, 128, 16, ctx, ctx[0], flash=flash)
+    assert sum(-(-n // 16) for n in ctx) * 8 > (2048 if flash else 4096) // 16 * grid
+
+
+def abi_call(args, out, ws):
+    """pkv_paged_attention of a pool_case's float16 arguments in a given workspace."""
+    q, k, v, table, ctx, Hkv, scale, bs, max_seq = args
+    B, Hq, D = q.shape
+    _lib.check(_lib.lib().pkv_paged_attention(
+        out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr(), ctx.data_ptr(), None, B, Hq, Hkv, D,
+        bs, table.shape[1], max_seq, k.shape[0], scale, q.stride(0), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
+        _lib.PKV_LAYOUT_PAGED5D, 0, ws.data_ptr(), ws.numel(), _lib.PKV_F16, _lib.PKV_F16, 1.0, 1.0,
+        torch.cuda.current_stream().cuda_stream))
+
+
+def test_workspace_without_room_for_pieces():
+    args, _, ref = pool_case("float16", "float16", 12, 6, 128, 16, CONTEXTS, 16384)
+    sizes = (len(CONTEXTS), 12, 6, 128, 16384, 0)
+    least = _lib.lib().pkv_paged_attention_workspace_size(*sizes)
+    full = _lib.lib().pkv_paged_attention_full_workspace_size(*sizes)
+    assert full > least
+    for nbytes, split in ((least, False), (full - 1, False), (full, True)):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+        out = torch.empty_like(args[0])
+        abi_call(args, out, ws)
+        assert any("split_kernel" in name for name, _ in kernels_of(lambda: abi_call(args, out, ws))) == split
+        atol, rtol = tolerance("float16", "float16")
+        np.testing.assert_allclose(to_f64(out), ref, atol=atol, rtol=rtol)
+        assert not ws[:_lib.PKV_COUNTER_BYTES].any()
