@@ -2059,6 +2059,16 @@ constexpr int kSplitWaves = 4;
 constexpr int kItemTiles = 16;
 constexpr int kMinPiece = 4;
 constexpr int kMinSpan = 16;
+// Longest context, in tiles, up to which each workgroup takes one whole item
+// (the host decides for this kernel by max_seq_len, which a captured graph may
+// hold far above its contexts): cutting such short items costs more than it
+// balances.  Device times, cut -> whole (the kernel that runs without the
+// split's room): 24 x 8 token rows of 300 .. 500 17.6 -> 13.0 us (17.3); bf16,
+// 3 x 16, D 96, of 100 .. 300 9.7 -> 7.8 (6.6), of 300 .. 500 10.6 -> 9.5
+// (8.4), at 500 .. 800 10.9 -> 11.8 (10.8).  kWholeOfPersist: in the persistent kernel's place
+// (44 x 8, bf16, D 128, of 500 .. 1000 32.6 -> 29.6 (27.4), of 1000 .. 2000
+// 51.4 -> 53.8 (47.1)).
+constexpr int kWholeTiles = 32, kWholeOfPersist = 64;
 // Most workgroups per item of the average length.
 constexpr int kMaxPieces = 32;
 // Tokens whose block (row) ids a workgroup holds at a time; longer pieces take
@@ -2071,31 +2081,43 @@ __device__ __forceinline__ int seq_tiles(const DecodeParams& p, uint32_t ctx) {
 }
 
 // s_pref[s]: the sum of (tiles + kItemTiles) over the sequences before s (of
-// one unit each), s_pref[B] the total; returns the span.  Every thread of the
-// workgroup calls it; needs B <= kPersistMaxOrder.
+// one unit each), s_pref[B] the total; returns the span, 0 where no context has
+// more than p.split_whole tiles and the grid has a workgroup for every item:
+// then each takes one whole item.  Every thread of the workgroup calls it;
+// needs B <= kPersistMaxOrder.  s_tmp: 2 NT / 64 ints.
 template <int NT>
-__device__ __forceinline__ int plan_spans(const DecodeParams& p, int32_t* s_pref, int32_t* s_tmp, int tid, int G) {
+__device__ __forceinline__ int plan_spans(const DecodeArgs& p, int32_t* s_pref, int32_t* s_tmp, int tid, int G) {
   constexpr int NW = NT / 64, PER = kPersistMaxOrder / NT;
   const int B = p.num_seqs;
   const int lane = tid & 63, wave = tid >> 6;
-  int v[PER], sum = 0;
+  int v[PER], sum = 0, longest = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int s = tid * PER + k;
-    v[k] = s < B ? seq_tiles(p, (uint32_t)p.context_lens[s]) + kItemTiles : 0;
+    const int n = s < B ? seq_tiles(p, (uint32_t)p.context_lens[s]) : -kItemTiles;
+    v[k] = n + kItemTiles;
     sum += v[k];
+    longest = max(longest, n);
   }
+  const bool more = __ballot(longest > p.split_whole) != 0;
   int incl = sum;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const int y = __shfl_up(incl, o);
     incl += lane >= o ? y : 0;
   }
-  if (lane == 63) s_tmp[wave] = incl;
+  if (lane == 63) {
+    s_tmp[wave] = incl;
+    s_tmp[NW + wave] = more;
+  }
   __syncthreads();
   int at = incl - sum;
+  bool whole = B * p.units <= G;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) at += w < wave ? s_tmp[w] : 0;
+  for (int w = 0; w < NW; ++w) {
+    at += w < wave ? s_tmp[w] : 0;
+    whole = whole && s_tmp[NW + w] == 0;
+  }
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int s = tid * PER + k;
@@ -2104,7 +2126,7 @@ __device__ __forceinline__ int plan_spans(const DecodeParams& p, int32_t* s_pref
   }
   if (tid == NT - 1) s_pref[kPersistMaxOrder] = at;
   __syncthreads();
-  return max((p.units * s_pref[B] + G - 1) / G, kMinSpan);
+  return whole ? 0 : max((p.units * s_pref[B] + G - 1) / G, kMinSpan);
 }
 
 // A place in the split schedule: tile `off` of item (seq, unit).
@@ -2114,6 +2136,10 @@ struct SplitPos {
 // Where workgroup w's span begins.  The span's own boundary is moved to an
 // item's start or end where it would leave a piece shorter than kMinPiece.
 __device__ __forceinline__ SplitPos split_pos(const int32_t* s_pref, int B, int units, int span, int w, int lane) {
+  if (span == 0) {
+    w = min(w, B * units);
+    return {w / units, w % units, 0};
+  }
   const int x = w * span;
   if (x >= units * s_pref[B]) return {B, 0, 0};
   // The last sequence that starts at or before x, in two steps of one lane each.
@@ -2239,7 +2265,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void paged_decode_split_kernel(De
   __shared__ float s_m[NW][16];
   __shared__ float s_l[NW][16];
   __shared__ int32_t s_pref[kPersistMaxOrder + 1];
-  __shared__ int32_t s_tmp[NW];
+  __shared__ int32_t s_tmp[2 * NW];
   __shared__ float2 s_ml[NT * 4 / D + 1];
   __shared__ int s_last;
   // Token rows: each wavefront's row ids (WaveRows).
@@ -2949,9 +2975,11 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
 //   448     14 of 4068 .. 4646 x 16, f32, D 64                  81.1    87.0
 //   648     27 of 8008 .. 9498 x 8, bf16, D 64                  95.9   101.6
 template <class QT, class CT, int D, int BS>
-static hipError_t launch_split(const DecodeArgs& p, int64_t other, hipStream_t stream, bool* launched) {
+static hipError_t launch_split(const DecodeArgs& args, int64_t other, hipStream_t stream, bool* launched) {
   *launched = false;
-  if (p.split_o == nullptr || p.num_seqs > kPersistMaxOrder) return hipSuccess;
+  if (args.split_o == nullptr || args.num_seqs > kPersistMaxOrder) return hipSuccess;
+  DecodeArgs p = args;
+  p.split_whole = other == 0 ? kWholeOfPersist : kWholeTiles;
   constexpr int64_t kTileBytes = (int64_t)kTile * D * 2 * Elem<CT>::kBytes;
   constexpr int64_t kMinTiles = BS == 0 ? 48 : (std::is_same<CT, F32>::value ? 1300000 : 1900000) / kTileBytes;  // per CU
   constexpr int NT = 64 * kSplitWaves;

@@ -125,6 +125,9 @@ struct DecodeArgs : DecodeParams {
   float* split_ml;
   float* split_o;
   int32_t* split_counters;
+  // Set by the launcher: the longest context, in tiles, of which every workgroup
+  // takes one whole item.
+  int32_t split_whole;
 };
 
 // The partition kernel merges its own partitions (the workgroup whose state

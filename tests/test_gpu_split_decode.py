@@ -3,8 +3,8 @@ contexts whose items are computed in pieces that workgroups merge.  Contexts
 around the tile and pass sizes, pieces longer than a pass, empty and over-long
 contexts between live ones, 16- and 32-bit and FP8 caches, token rows of one and
 of several tokens a block, explicit partition sizes, blocks outside the cache,
-a workspace without room for the pieces, a
-repeated call on the same scratch (arrival counters return to zero), and the
+contexts short enough for whole items, a workspace without room for the pieces,
+a repeated call on the same scratch (arrival counters return to zero), and the
 same result from run to run.  Every case checks that the kernel ran."""
 
 import numpy as np
@@ -211,3 +211,31 @@ def test_workspace_without_room_for_pieces():
         atol, rtol = tolerance("float16", "float16")
         np.testing.assert_allclose(to_f64(out), ref, atol=atol, rtol=rtol)
         assert not ws[:_lib.PKV_COUNTER_BYTES].any()
+
+
+@pytest.mark.parametrize("longest", [0, 31 * 16 + 1, 32 * 16, 32 * 16 + 1])
+def test_short_contexts_in_the_partition_kernel_s_place(longest):
+    # Whole items up to 32 tiles, pieces above.
+    ctx = [longest, 1, 0, 17, 500, 16385] + [min(longest, 100 * i) for i in range(1, 11)]
+    check("float16", "float16", 12, 6, 128, 16, ctx, 16384)
+    check("float16", "float16", 12, 6, 128, 16, ctx, 16384, flash=True)
+
+
+@pytest.mark.parametrize("longest", [64 * 16, 64 * 16 + 1])
+def test_short_contexts_in_the_persistent_kernel_s_place(longest):
+    # The same up to 64 tiles; 304 items.
+    ctx = [longest, 1, 0, 17, 500, 16385] + [5 * i for i in range(32)]
+    check("bfloat16", "bfloat16", 32, 8, 128, 16, ctx, 16384)
+
+
+@pytest.mark.parametrize("longest,whole", [(32 * 16, True), (32 * 16 + 1, False)])
+def test_whole_items_leave_no_pieces(longest, whole):
+    args, _, ref = pool_case("float16", "float16", 12, 6, 128, 16, [longest] * 16, 16384)
+    ws = torch.full((_lib.lib().pkv_paged_attention_full_workspace_size(16, 12, 6, 128, 16384, 0),), 77,
+                    dtype=torch.uint8, device="cuda")
+    ws[:_lib.PKV_COUNTER_BYTES].zero_()
+    out = torch.empty_like(args[0])
+    abi_call(args, out, ws)
+    atol, rtol = tolerance("float16", "float16")
+    np.testing.assert_allclose(to_f64(out), ref, atol=atol, rtol=rtol)
+    assert bool((ws[_lib.PKV_COUNTER_BYTES:] == 77).all()) == whole
