@@ -2968,7 +2968,27 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
 //   480     15 of 205 .. 3707 x 8, f32, D 256                  500.5   127.9
 //   384     24 of 500 .. 8000 x 8, f16 token rows, D 128       131.7    92.9
 //   416     26 of 789 .. 1869 x 8, bf16 token rows, D 80        41.7    33.4
-// and on the other side of the line:
+// and, device times of captured calls, on either side of the float32 line (1.3
+// MB a CU) and of the token rows' (48 tiles a CU):
+//   343     49 of 4189 .. 6982 x 1, f32, D 128 (1.4 MB)         81.7    62.9
+//   368     4 of 46631 x 4, f32, D 64 (1.5 MB)                  83.1    81.0
+//   264     22 of 13885 .. 23143 x 1, f32, D 64 (1.0 MB)        42.7    46.8
+//   368     46 of 1389 x 4, f32, D 64 (0.5 MB)                  26.3    31.9
+//   264     22 of 1427 .. 4757 x 4, rows, f16, D 256 (101)      68.8    57.8
+//   384     24 of 184 .. 3697 x 4, rows, f16, D 64 (85)         22.1    19.3
+//   336     28 of 1398 x 4, rows, f16, D 64 (38)                16.1    17.7
+//   432     3 of 8280 .. 9201 x 4, rows, f16, D 128 (27)        18.3    23.1
+// (below both lines uneven batches gain and nearly equal ones lose, up to a
+// quarter each; float32 at head size 256 gains throughout); of 8-token blocks,
+// the last four of the form that is left out (kNoGain):
+//   360     20 of 5316 .. 8861 x 1, f32, D 256                 142.6    64.5
+//   352     32 of 13160 .. 43868 x 1, FP8, D 192               124.7    67.7
+//   350     25 of 4358 .. 14528 x 2, f16, D 192                 95.1    72.2
+//   264     33 of 266 .. 5330 x 4, f16, D 256                  101.4    75.1
+//   336     56 of 225 .. 4510 x 2, f16, D 256                   53.9    52.9
+//   288     3 of 6866 .. 11142 x 16, f16, D 256                 82.0    84.9
+//   400     25 of 156 .. 3120 x 8, f16, D 256                   64.9    69.2
+// and on the other side of the grid's and the bytes' lines:
 //   256     2 of 4617 .. 8881 x 32, f32, D 128                  86.8    90.9
 //   256     16 of 256 .. 4096 x 8, bf16, D 128 (1.0 MB a CU)    31.7    32.4
 //   384     4 of 4745 .. 9063 x 32, bf16, D 64 (1.1 MB)         44.6    50.0
@@ -2977,27 +2997,37 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
 template <class QT, class CT, int D, int BS>
 static hipError_t launch_split(const DecodeArgs& args, int64_t other, hipStream_t stream, bool* launched) {
   *launched = false;
-  if (args.split_o == nullptr || args.num_seqs > kPersistMaxOrder) return hipSuccess;
-  DecodeArgs p = args;
-  p.split_whole = other == 0 ? kWholeOfPersist : kWholeTiles;
   constexpr int64_t kTileBytes = (int64_t)kTile * D * 2 * Elem<CT>::kBytes;
   constexpr int64_t kMinTiles = BS == 0 ? 48 : (std::is_same<CT, F32>::value ? 1300000 : 1900000) / kTileBytes;  // per CU
-  constexpr int NT = 64 * kSplitWaves;
-  static const int per_cu = resident_per_cu(paged_decode_split_kernel<QT, CT, D, BS>, NT);
-  const int64_t cus = device_cus();
-  const int64_t items = (int64_t)p.num_seqs * p.units;
-  const int64_t tiles = items * ((p.max_seq_len + kTile - 1) / kTile);
-  const int64_t grid = std::min<int64_t>({cus * per_cu, items * kMaxPieces, kSplitWorkgroups});
-  // (8-token blocks above head size 128: 3 of 6866 .. 11142 x 16, float16,
-  // D 256, 81.6 us, split 84.4.)
-  if (BS == 8 && D > 128) return hipSuccess;
-  const bool uneven = other == 0 || (BS == 0 ? other < 2 * cus : other > cus && 10 * other <= (D > 128 ? 20 : 17) * cus);
-  if (!uneven || grid < cus || items >= 2 * cus || tiles < cus * kMinTiles ||
-      tiles + items * kItemTiles + grid * kMinSpan > INT32_MAX)
-    return hipSuccess;
-  *launched = true;
-  hipLaunchKernelGGL((paged_decode_split_kernel<QT, CT, D, BS>), dim3((unsigned)grid), dim3(NT), 0, stream, p);
-  return hipGetLastError();
+  constexpr int kEven = D > 128 ? 20 : 17;  // tenths of a workgroup per CU
+  // 16-bit and FP8 caches of head sizes up to 64 never reach it: the partition
+  // kernel's grid is even before its partitions hold kMinTiles a CU, and of the
+  // persistent kernel two workgroups are resident per CU, so that it has
+  // two items for each.
+  constexpr bool kUnreached = BS > 0 && D <= 64 && !std::is_same<CT, F32>::value;
+  static_assert(!kUnreached || kMinTiles * 10 > (int64_t)kEven * (kMaxPartition / kTile), "partitions of kMinTiles");
+  // 8-token blocks of 16-bit caches at head size 256 gain on average no more
+  // than single batches lose.
+  constexpr bool kNoGain = BS == 8 && D > 192 && Elem<CT>::kBytes == 2;
+  if constexpr (!kUnreached && !kNoGain) {
+    if (args.split_o == nullptr || args.num_seqs > kPersistMaxOrder) return hipSuccess;
+    DecodeArgs p = args;
+    p.split_whole = other == 0 ? kWholeOfPersist : kWholeTiles;
+    constexpr int NT = 64 * kSplitWaves;
+    static const int per_cu = resident_per_cu(paged_decode_split_kernel<QT, CT, D, BS>, NT);
+    const int64_t cus = device_cus();
+    const int64_t items = (int64_t)p.num_seqs * p.units;
+    const int64_t tiles = items * ((p.max_seq_len + kTile - 1) / kTile);
+    const int64_t grid = std::min<int64_t>({cus * per_cu, items * kMaxPieces, kSplitWorkgroups});
+    const bool uneven = other == 0 || (BS == 0 ? other < 2 * cus : other > cus && 10 * other <= kEven * cus);
+    if (!uneven || grid < cus || items >= 2 * cus || tiles < cus * kMinTiles ||
+        tiles + items * kItemTiles + grid * kMinSpan > INT32_MAX)
+      return hipSuccess;
+    *launched = true;
+    hipLaunchKernelGGL((paged_decode_split_kernel<QT, CT, D, BS>), dim3((unsigned)grid), dim3(NT), 0, stream, p);
+    return hipGetLastError();
+  }
+  return hipSuccess;
 }
 
 template <class QT, class CT, int D, int BS>

@@ -155,21 +155,22 @@ def check(q, cache, Hq, Hkv, D, bs, ctx, max_seq_len, partition=0, **kw):
 
 
 @pytest.mark.parametrize("q", ["bfloat16", "float16", "float32"])
-@pytest.mark.parametrize("D,bs", [(128, 8), (128, 32), (256, 16), (256, 32)])
+@pytest.mark.parametrize("D,bs", [(128, 8), (128, 32), (256, 8), (256, 16), (192, 32)])
 def test_fp8(q, D, bs):
-    # Head size 256: in the partition kernel's place; 128: in the persistent
+    # Above head size 128 in the partition kernel's place; 128: in the persistent
     # kernel's (the line lies above what the partition kernel takes).
-    if D == 256:
+    if D > 128:
         check(q, FP8, 12, 6, D, bs, CONTEXTS, 16384)
     else:
         check(q, FP8, 16, 8, D, bs, [15000, 16, 1, 0, 9000, 4097, 16400] + [33] * 31, 16384)
 
 
-@pytest.mark.parametrize("q,cache", [("float16", "float16"), ("float32", "float32"), ("bfloat16", FP8)])
-@pytest.mark.parametrize("bs", [32, 16])
-def test_partition_sizes(q, cache, bs):
+@pytest.mark.parametrize("q,cache,D", [("float16", "float16", 192), ("float32", "float32", 256),
+                                       ("bfloat16", FP8, 256)])
+@pytest.mark.parametrize("bs", [8, 16])
+def test_partition_sizes(q, cache, D, bs):
     for partition in (512, 4096):
-        check(q, cache, 12, 6, 256, bs, CONTEXTS, 16384, partition=partition)
+        check(q, cache, 12, 6, D, bs, CONTEXTS, 16384, partition=partition)
 
 
 @pytest.mark.parametrize("bs", [8, 16, 32])
