@@ -123,11 +123,12 @@ size_t pkv_paged_attention_workspace_size(int32_t num_seqs, int32_t num_heads,
                                           int32_t max_seq_len,
                                           int32_t partition_size);
 
-/* Bytes of a workspace that lets pkv_paged_attention take every kernel it has:
- * at least the above, and room for the piece states of the split kernel, which
- * balances batches of few, long and uneven contexts over the chip.  With less
- * (but at least the above) such a batch runs the other kernels, to the same
- * result within rounding.  Returns 0 where the above does. */
+/* Bytes of a workspace that lets pkv_paged_attention take every kernel it has
+ * for these sizes on the current device: the above, or, where the sizes could
+ * take the split kernel, which balances batches of few, long and uneven contexts
+ * over the chip, also room for its piece states.  With less (but at least the
+ * above) such a batch runs the other kernels, to the same result within
+ * rounding.  Returns 0 where the above does. */
 size_t pkv_paged_attention_full_workspace_size(int32_t num_seqs, int32_t num_heads,
                                           int32_t num_kv_heads,
                                           int32_t head_size,

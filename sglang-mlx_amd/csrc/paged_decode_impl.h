@@ -44,7 +44,6 @@
 #pragma once
 
 #include <algorithm>
-#include <atomic>
 
 #include "pkv_fp8.h"
 #include "pkv_launch.h"
@@ -2905,22 +2904,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void paged_decode_reduce_kernel(D
 // Launchers
 // ---------------------------------------------------------------------------
 
-// Multiprocessor count of the current device, cached per device.
-// (Calls run in several threads at once: the cache is atomic, and the resident
-// workgroups of a kernel are static constants.)
-inline int device_cus() {
-  static std::atomic<int> cache[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
-// Workgroups of a kernel that one CU holds at once.
+// Workgroups of a kernel that one CU holds at once (called for static constants:
+// calls run in several threads at once).
 template <class Kernel>
 inline int resident_per_cu(Kernel kernel, int threads) {
   int n = 0;
@@ -2997,8 +2982,7 @@ static hipError_t launch_grouped(const DecodeParams& p, hipStream_t stream, bool
 template <class QT, class CT, int D, int BS>
 static hipError_t launch_split(const DecodeArgs& args, int64_t other, hipStream_t stream, bool* launched) {
   *launched = false;
-  constexpr int64_t kTileBytes = (int64_t)kTile * D * 2 * Elem<CT>::kBytes;
-  constexpr int64_t kMinTiles = BS == 0 ? 48 : (std::is_same<CT, F32>::value ? 1300000 : 1900000) / kTileBytes;  // per CU
+  constexpr int64_t kMinTiles = split_min_tiles(D, Elem<CT>::kBytes, BS == 0);
   constexpr int kEven = D > 128 ? 20 : 17;  // tenths of a workgroup per CU
   // 16-bit and FP8 caches of head sizes up to 64 never reach it: the partition
   // kernel's grid is even before its partitions hold kMinTiles a CU, and of the

@@ -232,7 +232,15 @@ size_t pkv_paged_attention_full_workspace_size(int32_t num_seqs, int32_t num_hea
                                                int32_t head_size, int32_t max_seq_len, int32_t partition_size) {
   const size_t least = pkv_paged_attention_workspace_size(num_seqs, num_heads, num_kv_heads, head_size, max_seq_len,
                                                           partition_size);
-  return least == 0 ? 0 : std::max(least, pkv::split_workspace_layout(num_heads, num_kv_heads, head_size).total);
+  if (least == 0 || num_seqs > pkv::kPersistMaxOrder) return least;
+  // Room for the pieces where a cache of some type and layout could take the
+  // split kernel at these sizes (launch_split).
+  const int64_t found = pkv::device_cus(), cus = found > 0 ? found : 256;
+  const int64_t items = (int64_t)num_seqs * num_kv_heads * ((num_heads / num_kv_heads + 15) / 16);
+  const int64_t tiles = items * (((int64_t)max_seq_len + pkv::kTile - 1) / pkv::kTile);
+  const int64_t line = std::min(pkv::split_min_tiles(head_size, 4, false), pkv::split_min_tiles(head_size, 2, true));
+  if (items >= 2 * cus || tiles < cus * line) return least;
+  return std::max(least, pkv::split_workspace_layout(num_heads, num_kv_heads, head_size).total);
 }
 
 size_t pkv_paged_attention_cascade_workspace_size(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,

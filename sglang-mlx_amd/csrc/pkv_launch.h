@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
 #include <type_traits>
 
 namespace pkv {
@@ -28,8 +29,26 @@ constexpr int kPersistMaxOrder = 1024;
 constexpr int persist_rows_max_seq(int head_size) { return head_size > 128 ? 2048 : 4096; }
 
 // Most workgroups of the split decode kernel (a state slot pair and a counter
-// each).
+// each), and the least tiles per CU that it is used from, were every context
+// max_seq_len long: 1.9 MB of tiles (1.3 MB of float32), 48 tiles of token rows.
 constexpr int kSplitWorkgroups = 1024;
+constexpr int64_t split_min_tiles(int head_size, int cache_elem, bool rows) {
+  return rows ? 48 : (cache_elem == 4 ? 1300000 : 1900000) / ((int64_t)kTile * head_size * 2 * cache_elem);
+}
+
+// Multiprocessor count of the current device, cached per device.
+// (Calls run in several threads at once: the cache is atomic.)  0: no device.
+inline int device_cus() {
+  static std::atomic<int> cache[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return (void)hipGetLastError(), 0;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
 
 struct RacParams {
   const void* key;

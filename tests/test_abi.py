@@ -187,6 +187,18 @@ def test_workspace_size_closed_form():
     assert lib.pkv_paged_attention_workspace_size(4, 28, 4, 128, 100, 8192) == 0
 
 
+@pytest.mark.parametrize("sizes,room", [
+    # (num_seqs, num_heads, num_kv_heads, head_size, max_seq_len)
+    ((1, 32, 8, 128, 1024), False), ((16, 32, 8, 128, 1024), False), ((64, 32, 8, 128, 16384), False),
+    ((2000, 4, 4, 128, 16384), False), ((24, 32, 8, 128, 8000), True), ((16, 6, 6, 256, 16384), True)])
+def test_room_for_pieces_only_where_the_split_kernel_could_run(sizes, room):
+    lib = _lib.lib()
+    least = lib.pkv_paged_attention_workspace_size(*sizes, 0)
+    full = lib.pkv_paged_attention_full_workspace_size(*sizes, 0)
+    assert full > least if room else full == least
+    assert lib.pkv_paged_attention_full_workspace_size(*sizes[:3], 0, sizes[4], 0) == 0
+
+
 def rac(**kw):
     a = dict(key=None, value=None, kc=None, vc=None, slots=None, N=4, H=8, D=128, ks=1024, vs=1024,
              layout=_lib.PKV_LAYOUT_PAGED5D, bs=16, x=8, num_slots=1024, kvd=_lib.PKV_BF16, cd=_lib.PKV_BF16,

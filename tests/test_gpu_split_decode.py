@@ -214,6 +214,36 @@ def test_workspace_without_room_for_pieces():
         assert not ws[:_lib.PKV_COUNTER_BYTES].any()
 
 
+@pytest.mark.parametrize("q,cache", [("float16", "float16"), ("float32", "float32"), ("float32", FP8)])
+@pytest.mark.parametrize("D", [32, 80, 128, 192, 256])
+def test_room_is_asked_for_wherever_the_kernel_runs(q, cache, D):
+    # The size's rule covers the launch's: sizes on either side of each line.
+    if cache == FP8 and D == 80:
+        D = 96
+    ran = 0
+    for B, Hkv, max_seq, flash in ((1, 8, 4096, False), (8, 1, 16384, True), (9, 8, 2730, True), (16, 6, 16384, False),
+                                   (12, 6, 5000, False), (33, 8, 16384, False), (63, 8, 4096, False),
+                                   (64, 8, 16384, False), (31, 1, 25000, False), (8, 8, 3072, True), (8, 8, 3056, True)):
+        if flash and cache != "float16":
+            continue
+        (qs, k, v, table, ctx, *_), _, _ = pool_case(q, cache, 2 * Hkv, Hkv, D, 16, [1] * B, max_seq, flash=flash, nb=4)
+        i = -2 if flash else 1
+        least = _lib.lib().pkv_paged_attention_workspace_size(B, 2 * Hkv, Hkv, D, max_seq, 0)
+        full = _lib.lib().pkv_paged_attention_full_workspace_size(B, 2 * Hkv, Hkv, D, max_seq, 0)
+        ws = torch.zeros(max(full, 64 << 20), dtype=torch.uint8, device="cuda")
+        code = {"float16": _lib.PKV_F16, "float32": _lib.PKV_F32, FP8: _lib.PKV_FP8_E4M3}
+        out = torch.empty_like(qs)
+        names = kernels_of(lambda: _lib.check(_lib.lib().pkv_paged_attention(
+            out.data_ptr(), qs.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr(), ctx.data_ptr(), None, B,
+            2 * Hkv, Hkv, D, 16, table.shape[1], max_seq, 4, 0.1, qs.stride(0), k.stride(0), k.stride(i), v.stride(0),
+            v.stride(i), _lib.PKV_LAYOUT_TOKEN_MAJOR if flash else _lib.PKV_LAYOUT_PAGED5D, 0, ws.data_ptr(),
+            ws.numel(), code[q], code[cache], 1.0, 1.0, torch.cuda.current_stream().cuda_stream)))
+        split = any("split_kernel" in n for n, _ in names)
+        ran += split
+        assert full > least or not split, (B, Hkv, max_seq, flash)
+    assert ran or cache == FP8 and D < 128
+
+
 @pytest.mark.parametrize("longest", [0, 31 * 16 + 1, 32 * 16, 32 * 16 + 1])
 def test_short_contexts_in_the_partition_kernel_s_place(longest):
     # Whole items up to 32 tiles, pieces above.
