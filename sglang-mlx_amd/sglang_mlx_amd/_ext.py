@@ -136,10 +136,11 @@ def _decode_scratch(dev: torch.device, stream: int, scratch_bytes: int) -> torch
             if held is None or held[0] != capture or held[1].numel() < scratch_bytes:
                 held = _ws_captured[key] = (capture, _new_scratch(dev, scratch_bytes))
             return held[1]
+        larger = _new_scratch(dev, scratch_bytes)
         if scratch is not None:
             _ws_outgrown.append(scratch)
-        scratch = _ws_cache[key] = _new_scratch(dev, scratch_bytes)
-        return scratch
+        _ws_cache[key] = larger
+        return larger
 
 
 def _cache_layout(key_cache, value_cache) -> int:

@@ -9,7 +9,7 @@ tensors: the reference's checks and messages in the reference's order
 import pytest
 import torch
 
-from sglang_mlx_amd import kernels
+from sglang_mlx_amd import _ext, kernels
 
 
 def pa_args(**kw):
@@ -197,3 +197,21 @@ def test_float32_caches():
     with pytest.raises(ValueError, match="float32 caches are read in the paged layout"):
         kernels.paged_attention_v1(**rows_args(query=q, key_cache=torch.zeros(96, 2, 64),
                                                value_cache=torch.zeros(96, 2, 64)))
+
+
+def test_scratch_that_cannot_grow_is_kept_once(monkeypatch):
+    # A failed allocation leaves the stream's scratch in use and lists nothing as outgrown.
+    old = torch.zeros(1 << 17, dtype=torch.uint8)
+    cache, outgrown = {(0, 5): old}, []
+    monkeypatch.setattr(_ext, "_ws_cache", cache)
+    monkeypatch.setattr(_ext, "_ws_outgrown", outgrown)
+    monkeypatch.setattr(_ext, "_native", type("N", (), {"capture_id": staticmethod(lambda stream: 0)}))
+
+    def fail(dev, scratch_bytes):
+        raise torch.OutOfMemoryError
+
+    monkeypatch.setattr(_ext, "_new_scratch", fail)
+    for _ in range(3):
+        with pytest.raises(torch.OutOfMemoryError):
+            _ext._decode_scratch(torch.device("cuda:0"), 5, 1 << 20)
+    assert cache == {(0, 5): old} and not outgrown
