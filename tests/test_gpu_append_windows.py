@@ -1,9 +1,11 @@
 """GPU parity of the paged append's window kernel, bit-exact over whole caches:
 whole-block runs at every offset of a window, runs broken at their first, a
 middle and their last token, the cache's last block, padding and slots past the
-cache, head sizes whose run tasks do not fill a workgroup, and FP8 codes whose
-quotients are ties, subnormals, overflows and zeros, at scales with and without
-an exact reciprocal and beyond the range of the corrected division."""
+cache, head sizes whose run tasks do not fill a workgroup, large calls whose
+workgroups take several heads, small ones on either side of the search for runs,
+and FP8 codes whose quotients are ties, subnormals, overflows and zeros, or come
+from every 16-bit pattern, at scales with and without an exact reciprocal and
+beyond the range of the corrected division."""
 
 import numpy as np
 import pytest
@@ -127,3 +129,43 @@ def test_small_calls_with_whole_blocks(bs, N, H, D, kv):
         at = [free.pop() for _ in range(min(-(-n // bs), len(free)))] if free else []
         slots += [b * bs + t for b in at for t in range(bs)][:n] if at else [-1] * n
     check(bs, H, D, kv, "float16" if kv == "float32" else kv, seed=N, nb=nb, slots=np.array(slots[:N], dtype=np.int32))
+
+
+def many_windows(bs, N, seed):
+    """(slots, blocks) of at least N tokens: window_slots over several parts of one cache."""
+    part, out = 3 * bs + 16, []
+    while sum(len(x) for x in out) < N:
+        s = window_slots(bs, part, seed + len(out))
+        out.append(np.where(s >= part * bs, 1 << 30, np.where(s < 0, -1, s + len(out) * part * bs)))
+    return np.concatenate(out).astype(np.int32), len(out) * part
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("H,D", [(7, 64), (3, 32), (5, 80), (2, 128), (9, 16)])
+@pytest.mark.parametrize("pair", [("bfloat16", "bfloat16"), ("float32", "float16"), ("bfloat16", FP8)])
+def test_large_calls_of_several_heads_a_workgroup(bs, H, D, pair):
+    # From 8192 (token, head) pairs on a workgroup takes a window of as many
+    # heads as give its threads a run task each; odd numbers of heads leave the
+    # last group short.
+    slots, nb = many_windows(bs, -(-8192 // H), seed=bs + D)
+    assert len(slots) * H >= 8192
+    check(bs, H, D, *pair, seed=3, scales=(0.05, 0.02) if pair[1] == FP8 else (1.0, 1.0), nb=nb, slots=slots)
+
+
+@pytest.mark.parametrize("kv_dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("scale", [1.0, 0.05, 0.02, -0.7, 1.0 / 3.0, 0.125, 2.0, 3e-3, 1e3, 7e-5, 2.0 ** -60, 2.0 ** 60,
+                                   1e-25])
+def test_fp8_codes_of_every_16_bit_pattern(kv_dtype, scale):
+    # 64 tokens x 8 heads x 128: half of the tokens fill blocks, half are scattered.
+    rng = np.random.default_rng(4)
+    key = np.arange(65536, dtype=np.uint16).reshape(64, 8, 128)
+    value = rng.permutation(65536).astype(np.uint16).reshape(64, 8, 128)
+    slots = np.concatenate([np.arange(32), 32 + rng.permutation(96)[:32]]).astype(np.int32)
+    kc0, vc0 = np.zeros((8, 8, 8, 16, 16), np.uint8), np.zeros((8, 8, 128, 16), np.uint8)
+    kc, vc = to_torch(kc0, FP8), to_torch(vc0, FP8)
+    kernels.reshape_and_cache(to_torch(key, kv_dtype), to_torch(value, kv_dtype), kc, vc, to_index(slots),
+                              k_scale=scale, v_scale=scale)
+    with np.errstate(all="ignore"):
+        rk, rv = orc.reshape_and_cache_paged5d(key, value, kc0, vc0, slots, kv_dtype, FP8, scale, scale)
+    np.testing.assert_array_equal(to_numpy(kc), rk)
+    np.testing.assert_array_equal(to_numpy(vc), rv)

@@ -59,16 +59,20 @@ def test_kernels_fit_lds_and_do_not_spill():
     # Every kernel's static LDS, as the runtime reports it, fits a workgroup;
     # the decode kernels of the hot path (16-bit queries at head sizes up to
     # 128: the persistent kernel in both its layouts, the grouped kernel,
-    # the cascade and the partition kernel) keep their registers out of
-    # scratch.  (Float32 queries and head sizes 192/256 do spill: 48-68
+    # the cascade, the partition and the split kernel) and the paged append's
+    # window kernel keep their registers out of scratch.  (Float32 queries and head sizes 192/256 do spill: 48-68
     # bytes in the grouped kernel, up to 284 in the float32 D256 kernels.)
     lds = _ext.get_max_shared_memory_per_block_device_attribute()
     attrs = kernel_attributes()
     assert len(attrs) > 100
     for k, a in attrs.items():
         assert a.sharedSizeBytes <= lds, (k, a.sharedSizeBytes)
-    hot = [k for k in attrs if re.search(r"(persist|group|cascade|part)_kernelINS_(4BF16|3F16)E", k)
+    hot = [k for k in attrs if re.search(r"(persist|group|cascade|part|split)_kernelINS_(4BF16|3F16)E", k)
            and not re.search(r"Li(192|256)E", k)]
+    split, window = [k for k in hot if "split_kernel" in k], [k for k in attrs if "rac_paged_window_kernel" in k]
+    assert any("Li128ELi0E" in k for k in split) and any("ENS_3FP8ELi128ELi16E" in k for k in split)
+    assert any("ENS_3FP8E" in k for k in window) and any("3F32ENS_3F16E" in k for k in window)
+    hot += window
     assert any("persist" in k and "Li128ELi0E" in k for k in hot)  # the token-row variant is covered
     assert any("group_kernel" in k for k in hot) and any("cascade_kernel" in k for k in hot)
     for k in hot:

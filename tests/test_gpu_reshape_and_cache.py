@@ -234,9 +234,9 @@ def test_large_append_of_slot_runs(kv_dtype, cache_dtype):
 @pytest.mark.parametrize("kv_dtype,cache_dtype", [("bfloat16", "bfloat16"), ("float32", "float16")])
 @pytest.mark.parametrize("head_dim", [64, 128, 256])
 def test_whole_block_runs(block_size, kv_dtype, cache_dtype, head_dim):
-    # Whole blocks written by consecutive tokens take the one-wavefront-per-
-    # (block, head) path; partial blocks, single slots and padding in the
-    # same batch take the per-token path.
+    # Whole blocks written by consecutive tokens are found by the workgroups of
+    # their windows and written as whole regions; partial blocks, single slots
+    # and padding in the same batch are written token by token.
     H = 4
     case = make_run_append_case(40 + block_size, N=600, H=H, D=head_dim, num_blocks=160, block_size=block_size,
                                 kv_dtype=kv_dtype, cache_dtype=cache_dtype)
