@@ -434,11 +434,13 @@ int paged_attention_impl(void* out, const void* query, const void* key_cache, co
                  max_seq_len <= (rows ? pkv::persist_rows_max_seq(head_size) : pkv::kPersistMaxSeq);
   // The split kernel needs its states' room, which a workspace of
   // pkv_paged_attention_workspace_size() bytes may lack; such calls run the
-  // other kernels.
+  // other kernels, as do a cascade's shapes that are decoded in one pass (its
+  // workspace is not sized for the pieces, and what a larger one would hold
+  // must not choose the kernel).
   const pkv::DecodeWorkspace sw = pkv::split_workspace_layout(num_heads, num_kv_heads, head_size);
   p.split_ml = p.split_o = nullptr;
   p.split_counters = reinterpret_cast<int32_t*>(ws);
-  if (workspace_bytes >= sw.total) {
+  if (plan == nullptr && workspace_bytes >= sw.total) {
     p.split_ml = reinterpret_cast<float*>(ws + pkv::kCounterBytes);
     p.split_o = reinterpret_cast<float*>(ws + pkv::kCounterBytes + sw.ml_bytes);
   }

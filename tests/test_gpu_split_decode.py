@@ -15,7 +15,8 @@ from oracle import pagedkv_oracle as orc
 from pkv_cases import X_OF, decode_oracle, make_decode_case, normal, tolerance
 from pkv_kernels import kernels_of
 from pkv_torch import to_f64, to_index, to_torch
-from sglang_mlx_amd import _lib, kernels
+from sglang_mlx_amd import _ext, _lib, kernels
+from sglang_mlx_amd.srt.mem_cache import build_cascade_plan
 
 pytestmark = pytest.mark.gpu
 FP8 = "fp8_e4m3"
@@ -270,3 +271,21 @@ def test_whole_items_leave_no_pieces(longest, whole):
     atol, rtol = tolerance("float16", "float16")
     np.testing.assert_allclose(to_f64(out), ref, atol=atol, rtol=rtol)
     assert bool((ws[_lib.PKV_COUNTER_BYTES:] == 77).all()) == whole
+
+
+def test_cascade_in_one_pass_does_not_depend_on_the_scratch():
+    # Head size 96 has no cascade kernel: the same bytes whatever scratch
+    # earlier calls of the stream left.
+    args, _, ref = pool_case("float16", "float16", 12, 6, 96, 16, [2000 - 90 * i for i in range(16)], 16384)
+    plan = build_cascade_plan(args[3].cpu().numpy(), args[4].cpu().numpy(), 16, 12, 6, device="cuda")
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        first = kernels.paged_attention_cascade(*args, plan)
+        assert _ext._ws_cache[(0, stream.cuda_stream)].numel() < 1 << 20
+        _ext._decode_scratch(args[0].device, stream.cuda_stream, 64 << 20)
+        again = kernels.paged_attention_cascade(*args, plan)
+    stream.synchronize()
+    atol, rtol = tolerance("float16", "float16")
+    np.testing.assert_allclose(to_f64(first), ref, atol=atol, rtol=rtol)
+    assert torch.equal(first, again)
