@@ -87,9 +87,10 @@ const char* pkv_last_error(void);
  *               F32 / F16 / BF16 -> PKV_FP8_E4M3.
  * k_scale, v_scale: FP8 caches store encode(x / k_scale) for keys and
  *               encode(x / v_scale) for values (the quantisation of
- *               convert_fp8.metal:33-35; both finite and nonzero; a
- *               power-of-two scale multiplies by its exact reciprocal, which
- *               is the same result).  FP8 caches need 16-byte aligned
+ *               convert_fp8.metal:33-35; both finite and nonzero; where both
+ *               magnitudes lie in [2^-60, 2^60] the quotients come from the
+ *               product with the rounded reciprocal and two correction
+ *               steps, to the same codes).  FP8 caches need 16-byte aligned
  *               key/value rows and caches, and x = 16 in the paged layout.
  *               Ignored for other caches (the reference has no FP8 append).
  */
@@ -109,8 +110,9 @@ int pkv_reshape_and_cache(const void* key, const void* value,
  * pairs and per-partition outputs (float32).  partition_size = 0 selects
  * the single-pass (v1) semantics; the library then chooses its own
  * schedule.  Zero-fill a workspace once, when it is allocated: its first
- * PKV_COUNTER_BYTES count the partitions of each (sequence, KV head) as
- * their workgroups finish, and every call leaves them zero again; the rest
+ * PKV_COUNTER_BYTES count the partitions of each (sequence, KV head), or the
+ * pieces of the split kernel (either layout), as their workgroups finish, and
+ * every call leaves them zero again; the rest
  * needs no initialisation (each launch reads only what it wrote).  Calls
  * ordered on one stream may share one workspace, also with
  * pkv_paged_attention_cascade; calls that overlap in time must not.
@@ -151,7 +153,8 @@ size_t pkv_paged_attention_full_workspace_size(int32_t num_seqs, int32_t num_hea
  *                      a multiple of 16 and of block_size, at most 4096.  A
  *                      workgroup takes a run of consecutive partitions (as
  *                      many as keep one workgroup per CU) and merges them as
- *                      it streams; the result is the same log-sum-exp merge.
+ *                      it streams, or the split kernel runs (below); the
+ *                      result is the same log-sum-exp merge.
  * Launches (all on `stream`): for partition_size = 0, contexts of at most
  * 16384 tokens and at least one (sequence, KV head) item per resident
  * workgroup, one persistent kernel that gives each item to one workgroup,
@@ -159,8 +162,14 @@ size_t pkv_paged_attention_full_workspace_size(int32_t num_seqs, int32_t num_hea
  * most 4 and contexts of at most 8192 tokens -- 4096 over FP8 caches at
  * head sizes 64 and 128 -- items of four sequences that share the MFMA
  * columns, so that tiles the four map to the same block are read once);
- * otherwise a partition kernel.  When a sequence has more than one
- * partition: with at most 8 partitions per sequence (paged layout, and
+ * otherwise a partition kernel.  In the place of either, for any
+ * partition_size, one split kernel where the workspace has room for it
+ * (pkv_paged_attention_full_workspace_size), there are fewer than two items
+ * per CU, max_seq_len gives each CU enough tokens and whole items or
+ * partitions would load the CUs unevenly: the items lie end to end, every
+ * workgroup takes an equal span of them, and the workgroup whose piece of an
+ * item arrives last merges its pieces, in a fixed order.  After the partition
+ * kernel, when a sequence has more than one partition: with at most 8 partitions per sequence (paged layout, and
  * num_seqs * num_kv_heads counters within the counter region), the
  * workgroup that finishes a sequence's last partition merges them (log-sum-
  * exp, in partition order: results do not depend on which workgroup
