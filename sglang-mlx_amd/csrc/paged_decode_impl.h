@@ -2066,7 +2066,8 @@ constexpr int kMinSpan = 16;
 // 3 x 16, D 96, of 100 .. 300 9.7 -> 7.8 (6.6), of 300 .. 500 10.6 -> 9.5
 // (8.4), at 500 .. 800 10.9 -> 11.8 (10.8).  kWholeOfPersist: in the persistent
 // kernel's place (44 x 8, bf16, D 128, of 500 .. 800 30.0 -> 26.0 (25.8), of
-// 1000 .. 2000 51.4 -> 53.8 (47.1)).
+// 1000 .. 2000 51.4 -> 53.8 (47.1)).  Longer contexts pay 0.1 to 0.2 us a launch
+// for the look at the lengths.
 constexpr int kWholeTiles = 32, kWholeOfPersist = 64;
 // Most workgroups per item of the average length.
 constexpr int kMaxPieces = 32;
